@@ -57,19 +57,14 @@ typedef struct {
 
 /* Projection GEMMs Y[N,M] = X[N,K] W^T. For few tokens (the eval, N <= 96)
  * the hand-written weight-streaming kernel reads the pre-tiled copy of the
- * weight (its time is the HBM stream of W). Up to 1000 tokens the
- * hand-tiled prefill kernel (gemm_wide, same tiled copy) takes every
- * projection: measured on MI355X against hipBLASLt on the plain rows, with
- * cold weights, for the 4B shapes at 256-800 tokens it took 0.69-0.98 of
- * the time for qkv and in_proj, 0.55-0.74 for o_proj / out_proj and
- * 0.52-0.61 for down_proj (the last two split over K into fp32 partials
- * that the residual add sums), and 0.65-0.89 for the gated gate|up + silu.
- * At 1024 tokens hipBLASLt was faster for in_proj (69-72 against 77 us), so
- * above 1000 tokens the projections go to hipBLASLt, except gate|up, which
- * stays on the kernel up to 2048 tokens (0.84-1.03 of hipBLASLt + silu_mul
- * there); above that hipBLASLt + silu_mul measured faster for gate|up: a 4B
- * eval of 2560 tokens 25.48 -> 25.09 ms, and the 9B request with its
- * 4096-token eval 155.6 -> 150.9 ms.
+ * weight (its time is the HBM stream of W). Above that the hand-tiled kernels
+ * (gemm_wide, gemm_block, same tiled copy) take every projection, at the tile
+ * and K split cujev_gemm_plan picks: measured on MI355X against hipBLASLt's
+ * heuristic choice on the plain rows, with cold weights, for the 4B and 9B
+ * shapes at 13 token counts from 384 to 12288, 0.60-1.09 of its time (mean
+ * 0.91) before the silu_mul launch that gate|up then also needs (101 us of
+ * 956 at 10752 tokens). hipBLASLt is left for shapes the tiled copy does not
+ * cover and for the LM head.
  * CUJEV_SMALL_GEMM=0 / CUJEV_WIDE_GEMM=0 send those shapes to hipBLASLt. */
 static int env_on(const char *name) {
     const char *e = getenv(name);
@@ -83,8 +78,6 @@ static int small_gemm_ok(int N, int M, int K) {
     return cached && N <= CUJEV_GEMM_SMALL_MAX_N && cujev_gemm_small_splits(M, K) > 0;
 }
 
-#define CUJEV_WIDE_GATED_MAX_N 2048
-#define CUJEV_WIDE_MAX_N 1000
 static int wide_gemm_on(void) {
     static int cached = -1;
     if (cached < 0)
@@ -97,8 +90,7 @@ static hipError_t proj_gemm(cujev_model *m, const bf16_t *X, const bf16_t *W, co
     if (Wt && small_gemm_ok(N, M, K))
         return k_gemm_small(X, K, Wt, N, M, K, 0, 1, Y, M, NULL, m->stream);
     int rg, ng, sp;
-    if (Wt && wide_gemm_on() && N <= CUJEV_WIDE_MAX_N &&
-        cujev_gemm_wide_plan(N, M, K, 0, 1, &rg, &ng, &sp) == 0)
+    if (Wt && wide_gemm_on() && cujev_gemm_plan(N, M, K, 0, 1, &rg, &ng, &sp) == 0)
         return k_gemm_wide(X, K, Wt, N, M, K, 0, rg, ng, 1, Y, M, NULL, m->stream);
     return k_gemm(m->gemm, X, W, Y, 0, N, M, K, m->stream);
 }
@@ -122,11 +114,11 @@ static hipError_t resid_gemm(cujev_model *m, const bf16_t *X, const bf16_t *W, c
         }
         return k_gemm_small(X, K, Wt, N, M, K, 0, 1, m->y, M, NULL, m->stream);
     }
-    if (Wt && wide_gemm_on() && N <= CUJEV_WIDE_MAX_N) {
+    if (Wt && wide_gemm_on()) {
         size_t cap = m->ypart_bytes / ((size_t)N * M * 4);
-        const int max_sp = cap > 8 ? 8 : (int)cap;
+        const int max_sp = cap > 8 ? 8 : cap < 1 ? 1 : (int)cap;
         int rg, ng, sp;
-        if (max_sp >= 1 && cujev_gemm_wide_plan(N, M, K, 0, max_sp, &rg, &ng, &sp) == 0) {
+        if (cujev_gemm_plan(N, M, K, 0, max_sp, &rg, &ng, &sp) == 0) {
             if (sp > 1) {
                 *y = NULL;
                 *yp = m->ypart;
@@ -146,8 +138,8 @@ static hipError_t gate_up_gemm(cujev_model *m, const cujev_layer *ly, int N, int
         return k_gemm_small(m->xb, H, ly->wt_gate_up, N, 2 * I, H, 1, 1, m->act, I, NULL,
                             m->stream);
     int rg, ng, sp;
-    if (ly->wt_gate_up && wide_gemm_on() && N <= CUJEV_WIDE_GATED_MAX_N &&
-        cujev_gemm_wide_plan(N, 2 * I, H, 1, 1, &rg, &ng, &sp) == 0)
+    if (ly->wt_gate_up && wide_gemm_on() &&
+        cujev_gemm_plan(N, 2 * I, H, 1, 1, &rg, &ng, &sp) == 0)
         return k_gemm_wide(m->xb, H, ly->wt_gate_up, N, 2 * I, H, 1, rg, ng, 1, m->act, I, NULL,
                            m->stream);
     hipError_t e = proj_gemm(m, m->xb, ly->w_gate_up, NULL, m->proj, N, 2 * I, H);

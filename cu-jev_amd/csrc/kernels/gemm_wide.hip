@@ -69,7 +69,7 @@ enum { GW_PLAIN = 0, GW_GATED = 1, GW_PART = 2 };
  * and the wave's registers fit without scratch; else as 4 waves of RG. Each
  * output is summed by one wave in the same k order either way. */
 constexpr bool gw_eight_waves(int rg, int ng, int mode) {
-    return rg % 2 == 0 && (mode != GW_GATED || rg % 4 == 0) && ng % 2 == 0 && !(rg == 4 && ng == 12);
+    return rg % 2 == 0 && (mode != GW_GATED || rg % 4 == 0) && ng % 2 == 0;
 }
 
 DEV __amdgpu_buffer_rsrc_t gw_rsrc(const void *base, uint32_t bytes) {
@@ -292,9 +292,9 @@ hipError_t launch_mode(int RG, int NG, dim3 grid, hipStream_t s, const bf16 *X, 
     CUJEV_GW_CASE(2, 8)
     CUJEV_GW_CASE(2, 12)
     CUJEV_GW_CASE(4, 6)
-    CUJEV_GW_CASE(4, 8)
+    if constexpr (MODE == GW_GATED)
+        CUJEV_GW_CASE(4, 8)
     CUJEV_GW_CASE(4, 10)
-    CUJEV_GW_CASE(4, 12)
     CUJEV_GW_CASE(6, 4)
     CUJEV_GW_CASE(6, 6)
     CUJEV_GW_CASE(6, 8)
@@ -317,58 +317,77 @@ extern "C" int cujev_gemm_wide_supported(int RG, int NG, int gated) {
     switch (RG) {
     case 2: return NG == 8 || NG == 12;
     case 3: return !gated && (NG == 8 || NG == 12);
-    case 4: return NG == 6 || NG == 8 || NG == 10 || NG == 12;
+    case 4: return NG == 6 || NG == 8 || NG == 10 || NG == 12 || NG == 16;
     case 6: return NG == 4 || NG == 6 || NG == 8;
     case 8: return NG == 4 || NG == 6;
     default: return 0;
     }
 }
 
-/* Estimated microseconds of a plan, a linear model fitted to measured
- * launches on MI355X (the 4B prefill shapes at 256-2048 tokens, every tile
- * and split, cold weights; mean error 7 %; on the GEMM time alone its pick
- * is the measured best in 32 of 35 shape/token cases and within 11 % in
- * the rest): per
+/* The tiles gemm_block.hip computes: 256 rows x 128 (ungated), 192 or 256
+ * tokens. Gated 256 x 128 stays here: 36.6 against 39.5 us for the 4B gate|up
+ * at 384 tokens, 112.0 against 117.5 for the 9B one at 611 (the others there:
+ * ungated 4 x 8 37.6 against 41.6 us, qkv at 611 tokens; gated 4 x 12 94.5
+ * against 107.5 us, gate|up at 1300). */
+static int block_tile(int RG, int NG, int gated) {
+    return RG == 4 && ((NG == 8 && !gated) || NG == 12 || NG == 16);
+}
+
+/* Estimated microseconds of a plan. For the tiles of this file a linear model
+ * fitted to measured launches on MI355X (the 4B prefill shapes at 256-2048
+ * tokens, every tile and split, cold weights; mean error 7 %): per
  * round of 256 workgroups, the MFMA cycles of one wave, the W and X bytes a
  * workgroup loads over its K range and the bytes its waves read from LDS,
  * plus a fixed cost per round; with splits, the fp32 partials' write and
- * the residual add's read of them (about 5 TB/s). */
+ * the residual add's read of them (about 5 TB/s). For gemm_block's tiles the
+ * measured time of a 32-k unit, which grows with the share of the CUs at
+ * work (0.505-0.64 us at 256 tokens, 0.41-0.48 at 192, 0.355-0.42 at 128),
+ * and a fixed 8 us per round (10 gated). Over the 4B and 9B shapes at 13 token
+ * counts from 384 to 12288 the pick takes 1.02 times the measured best on
+ * average and 1.14 at worst. */
 static double plan_us(int N, int M, int K, int gated, int RG, int NG, int S) {
     const int rows = gated ? M / 2 : M;
     const int bm = gated ? 32 * RG : 64 * RG;
     const long mb = (rows + bm - 1) / bm, nb = (N + 16 * NG - 1) / (16 * NG);
     const long items = mb * nb * S;
+    const double mb_part = S > 1 ? (double)S * N * M * 4 / 1e6 : 0.0;
+    if (block_tile(RG, NG, gated)) {
+        const double base = NG == 16 ? 0.505 : NG == 12 ? 0.41 : 0.355;
+        const double load = NG == 16 ? 0.135 : NG == 12 ? 0.07 : 0.065;
+        const double fixed = gated ? 10.0 : 8.0, units = (double)K / 32 / S;
+        const long full = items / 256, rem = items % 256;
+        double us = full * (units * (base + load) + fixed);
+        if (rem)
+            us += units * (base + load * rem / 256) + fixed;
+        return us + 0.3 * mb_part;
+    }
     const double rounds = (double)((items + 255) / 256);
     const double nch = (double)K / GW_KC / S;
     const double mfma = nch * 4 * RG * NG * 16;
     const double wbytes = nch * 16384.0 * RG;
     const double xbytes = nch * 256.0 * 16 * NG;
     const double lds = nch * 16384.0 * NG;
-    double us = rounds * (2.667e-4 * mfma + 8.406e-6 * wbytes + 1.016e-6 * xbytes +
-                          4.065e-6 * lds + 4.685);
-    if (S > 1) {
-        const double mb_part = (double)S * N * M * 4 / 1e6;
-        us += 0.1863 * mb_part + 0.2 * mb_part;
-    }
-    return us;
+    return rounds * (2.667e-4 * mfma + 8.406e-6 * wbytes + 1.016e-6 * xbytes + 4.065e-6 * lds +
+                     4.685) + 0.3863 * mb_part;
 }
 
-extern "C" int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *RG,
-                                    int *NG, int *S) {
+static int wide_plan(int N, int M, int K, int gated, int max_splits, int max_ng, int *RG, int *NG,
+                     int *S) {
     if (N <= 0 || M % 16 || K % GW_KC || (gated && M % 32))
         return -1;
     const char *force = getenv("CUJEV_WIDE_PLAN");
     if (force) {
         int a, b, c;
         if (sscanf(force, "%d,%d,%d", &a, &b, &c) == 3 && cujev_gemm_wide_supported(a, b, gated) &&
-            c >= 1 && c <= (max_splits < 1 ? 1 : max_splits) && (K / GW_KC) % c == 0) {
+            b <= max_ng && c >= 1 && c <= (max_splits < 1 ? 1 : max_splits) &&
+            (K / GW_KC) % c == 0) {
             *RG = a, *NG = b, *S = c;
             return 0;
         }
     }
     double best = 1e30;
     for (int rg = 2; rg <= 8; rg++)
-        for (int ng = 4; ng <= 12; ng += 2)
+        for (int ng = 4; ng <= max_ng; ng += 2)
             for (int s = 1; s <= (max_splits < 1 ? 1 : max_splits); s++) {
                 if (!cujev_gemm_wide_supported(rg, ng, gated) || (K / GW_KC) % s)
                     continue;
@@ -381,6 +400,16 @@ extern "C" int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_spli
     return best < 1e29 ? 0 : -1;
 }
 
+extern "C" int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *RG,
+                                    int *NG, int *S) {
+    return wide_plan(N, M, K, gated, max_splits, 12, RG, NG, S);
+}
+
+extern "C" int cujev_gemm_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG,
+                               int *S) {
+    return wide_plan(N, M, K, gated, max_splits, 16, RG, NG, S);
+}
+
 extern "C" hipError_t k_gemm_wide(const bf16_t *X, int ldx, const bf16_t *Wt, int N, int M, int K,
                                   int gated, int RG, int NG, int splits, bf16_t *Y, int ldy,
                                   float *P, hipStream_t stream) {
@@ -391,6 +420,11 @@ extern "C" hipError_t k_gemm_wide(const bf16_t *X, int ldx, const bf16_t *Wt, in
         (splits > 1 && !P) || (splits == 1 && !Y) ||
         (size_t)N * ldx * 2 > 0xffffffffull || (size_t)M * K * 2 > 0xffffffffull)
         return hipErrorInvalidValue;
+    if (block_tile(RG, NG, gated)) {
+        if (cujev_gemm_block_ok(X, ldx))
+            return k_gemm_block(X, ldx, Wt, N, M, K, gated, NG / 2, splits, Y, ldy, P, stream);
+        RG = 4, NG = 10; /* rows the DMA cannot take: another tile, the same bits */
+    }
     const int rows = gated ? M / 2 : M, bm = gated ? 32 * RG : 64 * RG;
     const int mblocks = (rows + bm - 1) / bm, nblocks = (N + 16 * NG - 1) / (16 * NG);
     const int items = mblocks * nblocks * splits, per_xcd = (items + 7) / 8;

@@ -296,10 +296,18 @@ hipError_t k_gemm_small_tile(const bf16_t *W, int M, int K, bf16_t *Wt, hipStrea
  * bf16 Y / gated act / fp32 partials P[splits][N][M]) for any N >= 1; M % 16
  * == 0 (gated: M % 32), K % 128 == 0, (K / 128) % splits == 0, X and W each
  * under 4 GiB. The tile is 64 RG weight rows (gated: 32 RG gate rows and the
- * same up rows) x 32 NG tokens; cujev_gemm_wide_plan picks RG, NG and a split
+ * same up rows) x 16 NG tokens; cujev_gemm_plan picks RG, NG and a split
  * count <= max_splits (1 = no partials) for a shape and returns 0, or -1 for
- * an unsupported shape. CUJEV_WIDE_PLAN="RG,NG,S" forces a plan. */
+ * an unsupported shape; cujev_gemm_wide_plan does so among the tiles of at
+ * most 192 tokens (the operator ABI's). CUJEV_WIDE_PLAN="RG,NG,S" forces a
+ * plan. Tiles (4, 8) ungated, (4, 12) and (4, 16) run in gemm_block.hip. */
+int cujev_gemm_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
 int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
+/* k_gemm_wide's 256-row tiles (gemm_block.hip): 32 WN tokens, WN 4, 6 or 8;
+ * _ok: whether X's rows can be loaded as 16-byte pieces. */
+int cujev_gemm_block_ok(const bf16_t *X, int ldx);
+hipError_t k_gemm_block(const bf16_t *X, int ldx, const bf16_t *Wt, int N, int M, int K, int gated,
+                        int WN, int splits, bf16_t *Y, int ldy, float *P, hipStream_t stream);
 int cujev_gemm_wide_supported(int RG, int NG, int gated);
 hipError_t k_gemm_wide(const bf16_t *X, int ldx, const bf16_t *Wt, int N, int M, int K, int gated,
                        int RG, int NG, int splits, bf16_t *Y, int ldy, float *P,

@@ -78,12 +78,13 @@ int cujev_ops_gemm_small_splits(int M, int K);
  * act[N][M/2], or fp32 partials P[splits][N][M] to be summed in split order)
  * through a hand-tiled MFMA kernel. M % 16 == 0 (gated: M % 32 == 0),
  * K % 128 == 0, (K/128) % splits == 0, X and W under 4 GiB each. The tile is
- * 64 rg weight rows (gated: 32 rg gate rows and the same up rows) x 32 ng
- * tokens; (rg, ng) must be a pair cujev_ops_gemm_wide_plan can return. */
+ * 64 rg weight rows (gated: 32 rg gate rows and the same up rows) x 16 ng
+ * tokens; (rg, ng) must be a pair cujev_ops_gemm_wide_plan can return, or
+ * (4, 16). Every pair gives the same bits. */
 int cujev_op_gemm_wide(const void *X, int ldx, const void *W, int N, int M, int K, int gated,
                        int rg, int ng, int splits, void *Y, int ldy, float *P, void *stream);
-/* The tile (rg, ng) and split count (<= max_splits) the engine uses for a
- * shape; 0 on success, -1 for an unsupported shape. */
+/* The best tile (rg, ng) of at most 192 tokens and split count (<=
+ * max_splits) for a shape; 0 on success, -1 for an unsupported shape. */
 int cujev_ops_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *rg, int *ng,
                              int *splits);
 
