@@ -313,7 +313,7 @@ cujev_status cujev_model_alloc_workspace(cujev_model *m) {
     /* + 8: a FUSED call's second (one-segment) chunk table heads */
     m->meta_ints = 3 * N + 3 * B + 4 * (size_t)m->max_chunks + B * (size_t)m->opts.max_candidates + B + 8;
     m->gemm_ws_bytes = (size_t)64 << 20;
-    m->attn_ws_bytes = cujev_attention_ws_max(m->max_tokens, m->Hq, m->Hkv);
+    m->attn_ws_bytes = cujev_attention_ws_max(m->max_tokens, m->Hkv);
     /* split-K partials: the few-token GEMM's at most 8 splits of 96 tokens,
      * and 64 MiB (or what 8 splits of all N tokens need, if less) for the
      * prefill GEMM, which fits its split count to it */

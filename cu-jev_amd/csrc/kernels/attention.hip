@@ -144,28 +144,47 @@ DEV void wait_lgkm(int n) { /* n is a constant once the loops are unrolled */
  * Per key tile i the loop overlaps, in each wave, the S^T MFMAs of tile i+1
  * with the softmax of tile i, then runs the PV MFMAs of tile i, while the
  * V^T of tile i+1 and the K of tile i+2 stream into the idle buffers. */
-/* Key-split partials (SPLIT): split s of a (token, q-head) row keeps the
- * unnormalised o[256], l and the shift mu of its share of the key tiles. */
+/* Key-split partials (SPLIT). The first `full` token tiles in launch order
+ * run in one pass (a launch of their own); each of the others is shared out
+ * over nsplit workgroups (blockIdx.y), and share sp of tile position pos and kv-head kh keeps, in slot
+ * ((pos - full) Hkv + kh) nsplit + sp, the unnormalised o[256], l and the
+ * shift mu of its share of the key tiles for its 4 x 32 (q-head, token) rows. */
 struct AttnPart {
-    float *o;  /* [nsplit][N][Hq][256] */
-    float *l;  /* [nsplit][N][Hq]      */
-    float *mu; /* [nsplit][N][Hq]      */
-    int nsplit;
+    float *o;  /* [slot][4][32][256] */
+    float *l;  /* [slot][4][32]      */
+    float *mu; /* [slot][4][32]      */
+    int nsplit, full;
 };
+constexpr int SLOT_ROWS = 4 * QW;
+
+/* Work mapping of block b of a one-pass grid: kv-head and position in launch
+ * order (>= the tile count: no work). The 8 XCDs are split among the
+ * kv-heads where Hkv divides 8. Position p serves token tile ntile - 1 - p. */
+DEV void block_work(int b, int Hkv, int *kh, int *pos) {
+    if (8 % Hkv == 0) {
+        const int G = 8 / Hkv, xcd = b & 7, slot = b >> 3;
+        *kh = xcd / G;
+        *pos = slot * G + xcd % G;
+    } else {
+        *kh = b % Hkv;
+        *pos = b / Hkv;
+    }
+}
 
 /* The second problem of a paired launch: N packed tokens starting row0
- * rows after the first problem's, over the shared state cache's first P
+ * rows from the first problem's, over the shared state cache's first P
  * keys and their own keys in (ok, ovt) (see k_attention). */
 struct AttnJob {
     const bf16 *ok, *ovt;
-    int row0, P, o_stride, N;
+    ptrdiff_t row0;
+    int P, o_stride, N;
 };
 
 /* PAIR (attention_pair): workgroups [0, nblk_a) serve the problem of the
  * leading arguments, the rest a second one over the same state cache, given
- * by jb (its rows start jb.row0 rows further into q, gate, own_base and
- * out; nblk_a is a multiple of 8 where Hkv divides 8, so both keep the XCD
- * mapping). Without PAIR, jb and nblk_a are unused. */
+ * by jb (its rows start jb.row0 rows from the first's in q, gate, own_base
+ * and out; nblk_a is a multiple of 8 where Hkv divides 8, so both keep the
+ * XCD mapping). Without PAIR, jb and nblk_a are unused. */
 template <bool SPLIT, bool PAIR>
 __global__ __launch_bounds__(256) void attention_kernel(
     const bf16 *__restrict__ q, const bf16 *__restrict__ gate, int gts, int ghs,
@@ -177,27 +196,21 @@ __global__ __launch_bounds__(256) void attention_kernel(
     int bid = blockIdx.x;
     if (PAIR && bid >= nblk_a) {
         bid -= nblk_a;
-        q += (size_t)jb.row0 * Hq * D, gate += (size_t)jb.row0 * gts;
-        own_base += jb.row0, out += (size_t)jb.row0 * Hq * D;
+        q += jb.row0 * Hq * D, gate += jb.row0 * gts;
+        own_base += jb.row0, out += jb.row0 * Hq * D;
         P = jb.P, ok = jb.ok, ovt = jb.ovt, o_stride = jb.o_stride, N = jb.N;
         ntile = (N + QW - 1) / QW;
     }
 
-    /* ---- XCD-aware work mapping ---- */
+    /* ---- XCD-aware work mapping ---- (SPLIT: the blocks past the whole
+     * tiles', a multiple of 8 where Hkv divides 8, once per share) */
     int kh, tile;
-    {
-        if (8 % Hkv == 0) {
-            const int G = 8 / Hkv, xcd = bid & 7, slot = bid >> 3;
-            kh = xcd / G;
-            tile = slot * G + xcd % G;
-        } else {
-            kh = bid % Hkv;
-            tile = bid / Hkv;
-        }
-        if (tile >= ntile)
-            return;
-        tile = ntile - 1 - tile;
-    }
+    block_work(SPLIT ? bid + part.full * Hkv : bid, Hkv, &kh, &tile);
+    if (tile >= ntile)
+        return;
+    const int split = SPLIT ? (int)blockIdx.y : 0;
+    const int slot = SPLIT ? ((tile - part.full) * Hkv + kh) * part.nsplit + split : 0;
+    tile = ntile - 1 - tile;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int head = kh * 4 + wave;
     const int h = lane >> 5, col = lane & 31;
@@ -224,14 +237,13 @@ __global__ __launch_bounds__(256) void attention_kernel(
     const int own_t0 = own_lo / BK;
     const int ntl_all = nst + own_hi / BK - own_t0 + 1;
     /* SPLIT: this workgroup's contiguous share [tb, tb + ntl) of the tiles */
-    const int split = SPLIT ? (int)blockIdx.y : 0;
     const int tb = SPLIT ? split * ntl_all / part.nsplit : 0;
     const int ntl = SPLIT ? (split + 1) * ntl_all / part.nsplit - tb : ntl_all;
+    const int prow = slot * SLOT_ROWS + wave * QW + col; /* partial row */
     if (SPLIT && ntl <= 0) { /* no tiles: an empty partial */
         if (qvalid && h == 0) {
-            const size_t r = ((size_t)split * N + n) * Hq + head;
-            part.l[r] = 0.f;
-            part.mu[r] = 0.f;
+            part.l[prow] = 0.f;
+            part.mu[prow] = 0.f;
         }
         return;
     }
@@ -493,8 +505,7 @@ __global__ __launch_bounds__(256) void attention_kernel(
         return;
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
     if constexpr (SPLIT) { /* the unnormalised partial; the merge gates it */
-        const size_t r = ((size_t)split * N + n) * Hq + head;
-        float *po = part.o + r * D;
+        float *po = part.o + (size_t)prow * D;
 #pragma unroll
         for (int dt = 0; dt < 8; dt++)
 #pragma unroll
@@ -503,8 +514,8 @@ __global__ __launch_bounds__(256) void attention_kernel(
                     make_float4(o[dt][4 * gq], o[dt][4 * gq + 1], o[dt][4 * gq + 2],
                                 o[dt][4 * gq + 3]);
         if (h == 0) {
-            part.l[r] = l_tot;
-            part.mu[r] = mu_run;
+            part.l[prow] = l_tot;
+            part.mu[prow] = mu_run;
         }
         return;
     }
@@ -529,16 +540,21 @@ __global__ __launch_bounds__(256) void attention_kernel(
 /* Merge of the key-split partials: per (token, q-head) row, with mu the
  * largest shift among the splits that saw keys, o = sum_s 2^(mu_s - mu) o_s
  * and l likewise (the same p = 2^(s - mu) for every split, up to fp32 sum
- * order); out = o / l * sigmoid(gate). One wave per row, 4 dims a lane. */
+ * order); out = o / l * sigmoid(gate). One wave per row, 4 dims a lane; 32
+ * workgroups per shared (tile, kv-head). */
 __global__ __launch_bounds__(256) void attention_merge_kernel(AttnPart part,
                                                               const bf16 *__restrict__ gate,
                                                               int gts, int ghs, int N, int Hq,
+                                                              int Hkv, int ntile,
                                                               bf16 *__restrict__ out) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (row >= N * Hq)
+    const int unit = blockIdx.x >> 5, lane = threadIdx.x & 63;
+    const int wrow = (blockIdx.x & 31) * 4 + (threadIdx.x >> 6); /* q-head of the group, token */
+    const int kh = unit % Hkv, tile = ntile - 1 - (part.full + unit / Hkv);
+    const int n = tile * QW + (wrow & (QW - 1)), head = kh * 4 + wrow / QW;
+    if (n >= N)
         return;
-    const int n = row / Hq, head = row % Hq;
-    const size_t rs = (size_t)N * Hq;
+    const int row = n * Hq + head;
+    const size_t r0 = (size_t)unit * part.nsplit * SLOT_ROWS + wrow;
     /* every split's l, mu and o slice in flight before any arithmetic */
     float ls[CUJEV_ATTN_MAX_SPLITS], ms[CUJEV_ATTN_MAX_SPLITS];
     float4 os[CUJEV_ATTN_MAX_SPLITS];
@@ -546,9 +562,10 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnPart part,
     for (int sp = 0; sp < CUJEV_ATTN_MAX_SPLITS; sp++) {
         ls[sp] = 0.f, ms[sp] = 0.f, os[sp] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (sp < part.nsplit) { /* uniform */
-            ls[sp] = part.l[sp * rs + row];
-            ms[sp] = part.mu[sp * rs + row];
-            os[sp] = *(const float4 *)(part.o + (sp * rs + row) * D + 4 * lane);
+            const size_t r = r0 + (size_t)sp * SLOT_ROWS;
+            ls[sp] = part.l[r];
+            ms[sp] = part.mu[r];
+            os[sp] = *(const float4 *)(part.o + r * D + 4 * lane);
         }
     }
     float mu = -INFINITY;
@@ -763,27 +780,61 @@ extern "C" hipError_t k_attn_prep_pair(const bf16_t *proj, int proj_stride,
     return hipGetLastError();
 }
 
-extern "C" int cujev_attention_splits(int N, int Hkv, int P) {
-    const int wgs = CEIL_DIV(N, QW) * Hkv;
+/* How a shape is shared out: token tiles 0 .. *full - 1 in launch order run
+ * whole, the rest over the returned number of workgroups each (1: no split).
+ * Whole rounds of 256 workgroups stay whole; what is left over (everything,
+ * when there is less than one round) is split so that at most 256 workgroups
+ * run it: at 64 branches x 40 over 8192 keys the last 64 of 320 workgroups
+ * would otherwise hold a second round of 130 key tiles on a quarter of the
+ * CUs. A split pays where the key tiles it takes off the longest share, at
+ * about 1.5 us each, exceed the partials' write and read (0.3 us per MB) and
+ * the merge launch (6 us); the smallest evals (N <= 256 tokens, under 128
+ * workgroups) always split, as measured there. Every split needs at most 256
+ * slots of partials. */
+extern "C" int cujev_attention_splits(int N, int Hkv, int P, int *full) {
+    *full = 0;
+    if (N <= 0 || P < 0 || Hkv <= 0)
+        return 1;
+    const int ntile = CEIL_DIV(N, QW);
     /* at most as many shares as a token tile has key tiles (state + own) */
     const int ntl_max = CEIL_DIV(P, BK) + CEIL_DIV(N, BK) + 1;
-    if (N <= 0 || P < 0 || N > CUJEV_ATTN_SPLIT_MAX_N || wgs >= 128)
+    if (N <= CUJEV_ATTN_SPLIT_MAX_N && ntile * Hkv < 128) {
+        int s = 256 / (ntile * Hkv);
+        s = s > ntl_max ? ntl_max : s;
+        s = s > CUJEV_ATTN_MAX_SPLITS ? CUJEV_ATTN_MAX_SPLITS : s;
+        return s < 1 ? 1 : s;
+    }
+    const int nf = ntile * Hkv / 256 * 256 / Hkv; /* tiles of the whole rounds */
+    const int units = (ntile - nf) * Hkv;
+    if (units <= 0 || units > 128)
         return 1;
-    int s = 256 / wgs;
-    s = s > ntl_max ? ntl_max : s;
-    s = s > CUJEV_ATTN_MAX_SPLITS ? CUJEV_ATTN_MAX_SPLITS : s;
-    return s < 1 ? 1 : s;
+    /* key tiles of the longest leftover tile: the state and about two of its
+     * own; with no state a causal prefill's, whose last positions are short */
+    const int len = P > 0 ? CEIL_DIV(P, BK) + 2 : (ntile - nf) * QW / BK + 1;
+    int best = 1;
+    double best_us = 1.5 * len;
+    for (int s = 2; s <= 256 / units && s <= CUJEV_ATTN_MAX_SPLITS && s <= len; s++) {
+        const double us = 1.5 * CEIL_DIV(len, s) + 6.0 + 0.3 * 0.132 * units * s;
+        if (us < best_us)
+            best_us = us, best = s;
+    }
+    if (best > 1)
+        *full = nf;
+    return best;
 }
 
-extern "C" size_t cujev_attention_ws_bytes(int N, int Hq, int nsplit) {
-    return nsplit > 1 ? (size_t)nsplit * N * Hq * (D + 2) * sizeof(float) : 0;
+/* Bytes of the partials of a shape; 0 when it does not split. */
+extern "C" size_t cujev_attention_ws_bytes(int N, int Hkv, int P) {
+    int full;
+    const int s = cujev_attention_splits(N, Hkv, P, &full);
+    return s > 1 ? (size_t)(CEIL_DIV(N, QW) - full) * Hkv * s * SLOT_ROWS * (D + 2) * sizeof(float)
+                 : 0;
 }
 
-extern "C" size_t cujev_attention_ws_max(int max_tokens, int Hq, int Hkv) {
+extern "C" size_t cujev_attention_ws_max(int max_tokens, int Hkv) {
     size_t best = 0;
-    const int nmax = max_tokens < CUJEV_ATTN_SPLIT_MAX_N ? max_tokens : CUJEV_ATTN_SPLIT_MAX_N;
-    for (int n = 1; n <= nmax; n++) { /* P large: the most shares */
-        const size_t b = cujev_attention_ws_bytes(n, Hq, cujev_attention_splits(n, Hkv, 1 << 20));
+    for (int n = 1; n <= max_tokens; n++) { /* P large: the most shares */
+        const size_t b = cujev_attention_ws_bytes(n, Hkv, 1 << 20);
         best = b > best ? b : best;
     }
     return best;
@@ -811,21 +862,33 @@ extern "C" hipError_t k_attention(const bf16_t *q, const bf16_t *gate, int gate_
         return hipErrorInvalidValue;
     const int ntile = CEIL_DIV(N, QW);
     const int nblk = attention_blocks(ntile, Hkv);
-    /* Few workgroups (an eval of a few branches: 4 kv-heads x 3 token tiles
-     * at 80 tokens): split the key tiles over blockIdx.y so that about 256
-     * workgroups run, when the workspace holds the partials. */
-    const int nsplit = cujev_attention_splits(N, Hkv, P);
-    if (nsplit > 1 && ws && ws_bytes >= cujev_attention_ws_bytes(N, Hq, nsplit)) {
-        const size_t rows = (size_t)nsplit * N * Hq;
-        AttnPart part{(float *)ws, (float *)ws + rows * D, (float *)ws + rows * (D + 1), nsplit};
-        hipLaunchKernelGGL((attention_kernel<true, false>), dim3((unsigned)nblk, (unsigned)nsplit),
-                           dim3(256), 0, stream, (const bf16 *)q, (const bf16 *)gate,
-                           gate_tok_stride, gate_head_stride, (const bf16 *)pk, (const bf16 *)pvt,
-                           P, p_stride, (const bf16 *)ok, (const bf16 *)ovt, o_stride, own_base, N,
-                           Hq, Hkv, ntile, (bf16 *)out, part, AttnJob{}, 0);
-        hipLaunchKernelGGL(attention_merge_kernel, dim3((unsigned)CEIL_DIV(N * Hq, 4)), dim3(256),
-                           0, stream, part, (const bf16 *)gate, gate_tok_stride, gate_head_stride,
-                           N, Hq, (bf16 *)out);
+    /* Workgroups that do not fill a round share out their key tiles, when
+     * the workspace holds the partials. */
+    int full;
+    const int nsplit = cujev_attention_splits(N, Hkv, P, &full);
+    if (nsplit > 1 && ws && ws_bytes >= cujev_attention_ws_bytes(N, Hkv, P)) {
+        const int units = (ntile - full) * Hkv;
+        const size_t rows = (size_t)units * nsplit * SLOT_ROWS;
+        AttnPart part{(float *)ws, (float *)ws + rows * D, (float *)ws + rows * (D + 1), nsplit,
+                      full};
+        /* The whole rounds and the shares are two launches: one kernel doing
+         * both spilled 17 registers, and either launch fills the CUs. */
+        if (full > 0)
+            hipLaunchKernelGGL((attention_kernel<false, false>), dim3((unsigned)(full * Hkv)),
+                               dim3(256), 0, stream, (const bf16 *)q, (const bf16 *)gate,
+                               gate_tok_stride, gate_head_stride, (const bf16 *)pk,
+                               (const bf16 *)pvt, P, p_stride, (const bf16 *)ok,
+                               (const bf16 *)ovt, o_stride, own_base, N, Hq, Hkv, ntile,
+                               (bf16 *)out, AttnPart{}, AttnJob{}, 0);
+        hipLaunchKernelGGL((attention_kernel<true, false>),
+                           dim3((unsigned)(nblk - full * Hkv), (unsigned)nsplit), dim3(256), 0,
+                           stream, (const bf16 *)q, (const bf16 *)gate, gate_tok_stride,
+                           gate_head_stride, (const bf16 *)pk, (const bf16 *)pvt, P, p_stride,
+                           (const bf16 *)ok, (const bf16 *)ovt, o_stride, own_base, N, Hq, Hkv,
+                           ntile, (bf16 *)out, part, AttnJob{}, 0);
+        hipLaunchKernelGGL(attention_merge_kernel, dim3((unsigned)(units * 32)), dim3(256), 0,
+                           stream, part, (const bf16 *)gate, gate_tok_stride, gate_head_stride, N,
+                           Hq, Hkv, ntile, (bf16 *)out);
         return hipGetLastError();
     }
     hipLaunchKernelGGL((attention_kernel<false, false>), dim3((unsigned)nblk), dim3(256), 0, stream,
@@ -853,12 +916,27 @@ extern "C" hipError_t k_attention_pair(const bf16_t *q, const bf16_t *gate, int 
     if (Hq != 4 * Hkv || Pa < 0 || Pb < 0 || p_stride % 64 || oa_stride % 64 || ob_stride % 64)
         return hipErrorInvalidValue;
     const int ta = CEIL_DIV(Na, QW), tb = CEIL_DIV(Nb, QW);
-    const AttnJob jb{(const bf16 *)okb, (const bf16 *)ovtb, Na, Pb, ob_stride, Nb};
     const int na = attention_blocks(ta, Hkv), nb = attention_blocks(tb, Hkv);
+    const bf16 *q_ = (const bf16 *)q, *g_ = (const bf16 *)gate;
+    bf16 *o_ = (bf16 *)out;
+    /* The problem with the longer workgroups goes first, so that none of them
+     * starts when the others are done (64 branches x 40 after a prefill of
+     * 8192: the branches' 130 key tiles each behind the prefill's short last
+     * tiles took 1037 us). */
+    if (CEIL_DIV(Pb, BK) + 2 >= CEIL_DIV(Pa, BK) + CEIL_DIV(Na, BK)) {
+        const AttnJob ja{(const bf16 *)oka, (const bf16 *)ovta, -(ptrdiff_t)Na, Pa, oa_stride, Na};
+        hipLaunchKernelGGL((attention_kernel<false, true>), dim3((unsigned)(na + nb)), dim3(256),
+                           0, stream, q_ + (size_t)Na * Hq * D, g_ + (size_t)Na * gate_tok_stride,
+                           gate_tok_stride, gate_head_stride, (const bf16 *)pk, (const bf16 *)pvt,
+                           Pb, p_stride, (const bf16 *)okb, (const bf16 *)ovtb, ob_stride,
+                           own_base + Na, Nb, Hq, Hkv, tb, o_ + (size_t)Na * Hq * D, AttnPart{},
+                           ja, nb);
+        return hipGetLastError();
+    }
+    const AttnJob jb{(const bf16 *)okb, (const bf16 *)ovtb, Na, Pb, ob_stride, Nb};
     hipLaunchKernelGGL((attention_kernel<false, true>), dim3((unsigned)(na + nb)), dim3(256), 0,
-                       stream, (const bf16 *)q, (const bf16 *)gate, gate_tok_stride,
-                       gate_head_stride, (const bf16 *)pk, (const bf16 *)pvt, Pa, p_stride,
-                       (const bf16 *)oka, (const bf16 *)ovta, oa_stride, own_base, Na, Hq, Hkv, ta,
-                       (bf16 *)out, AttnPart{}, jb, na);
+                       stream, q_, g_, gate_tok_stride, gate_head_stride, (const bf16 *)pk,
+                       (const bf16 *)pvt, Pa, p_stride, (const bf16 *)oka, (const bf16 *)ovta,
+                       oa_stride, own_base, Na, Hq, Hkv, ta, o_, AttnPart{}, jb, na);
     return hipGetLastError();
 }

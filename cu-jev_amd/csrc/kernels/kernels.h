@@ -74,17 +74,18 @@ hipError_t k_attention(const bf16_t *q, const bf16_t *gate, int gate_tok_stride,
                        int p_stride, const bf16_t *ok, const bf16_t *ovt, int o_stride,
                        const int32_t *own_base, int N, int Hq, int Hkv, bf16_t *out,
                        void *ws, size_t ws_bytes, hipStream_t stream);
-/* With few workgroups (N <= CUJEV_ATTN_SPLIT_MAX_N tokens giving under 128
- * of them), k_attention splits the key tiles over
- * cujev_attention_splits() workgroups per token tile and merges their
- * softmax partials in a second kernel, when `ws` holds
- * cujev_attention_ws_bytes() bytes; otherwise (ws NULL) one pass. */
-#define CUJEV_ATTN_SPLIT_MAX_N 256
+/* Workgroups that do not fill a round of 256 (all of a small eval's, the last
+ * 64 of 320) share out their key tiles over cujev_attention_splits()
+ * workgroups per token tile (all but the first *full tiles in launch order)
+ * and a second kernel merges their softmax partials, when `ws` holds
+ * cujev_attention_ws_bytes() bytes (at most 32.25 MiB); otherwise (ws NULL)
+ * one pass. */
+#define CUJEV_ATTN_SPLIT_MAX_N 256 /* always split up to here, by cost above */
 #define CUJEV_ATTN_MAX_SPLITS 16
-int cujev_attention_splits(int N, int Hkv, int P);
-size_t cujev_attention_ws_bytes(int N, int Hq, int nsplit);
+int cujev_attention_splits(int N, int Hkv, int P, int *full);
+size_t cujev_attention_ws_bytes(int N, int Hkv, int P);
 /* the largest workspace any N <= max_tokens can use */
-size_t cujev_attention_ws_max(int max_tokens, int Hq, int Hkv);
+size_t cujev_attention_ws_max(int max_tokens, int Hkv);
 /* Two k_attention problems over one state cache (pk, pvt) in one launch,
  * one pass each (no key split): rows [0, Na) of q, gate, own_base and out
  * are problem a (the cache's first Pa keys, own keys in oka / ovta), rows

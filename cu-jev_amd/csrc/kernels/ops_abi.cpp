@@ -208,7 +208,8 @@ EXPORT int cujev_op_attention_pair(const void *q, const void *gate, int gate_tok
 }
 
 EXPORT size_t cujev_ops_attention_ws_bytes(int N, int Hq, int Hkv, int P) {
-    return cujev_attention_ws_bytes(N, Hq, cujev_attention_splits(N, Hkv, P));
+    (void)Hq; /* 4 Hkv */
+    return cujev_attention_ws_bytes(N, Hkv, P);
 }
 
 EXPORT int cujev_op_attention_ws(const void *q, const void *gate, int gate_tok_stride,
@@ -269,7 +270,7 @@ EXPORT int cujev_op_attention_noalloc(const void *q, const void *gate, int gate_
                                       int Hkv, void *out, void *stream) {
     if (N < 0 || P < 0 || Hkv <= 0)
         return fail(1, "attention_noalloc: bad arguments");
-    const size_t need = cujev_attention_ws_bytes(N, Hq, cujev_attention_splits(N, Hkv, P));
+    const size_t need = cujev_attention_ws_bytes(N, Hkv, P);
     if (need > CUJEV_OPS_ATTN_NOALLOC_SCRATCH_BYTES)
         return fail(6,
                     "attention_noalloc: N=%d, Hq=%d, Hkv=%d, P=%d needs %zu bytes of key-split "

@@ -148,9 +148,10 @@ int cujev_op_attention_pair(const void *q, const void *gate, int gate_tok_stride
                             const void *oka, const void *ovta, int oa_stride, int Nb, int Pb,
                             const void *okb, const void *ovtb, int ob_stride, void *stream);
 /* The same with a device workspace (no counterpart in the reference, whose
- * kernel has one pass): with few workgroups (N <= 256 tokens giving under
- * 128 of them) the key tiles are split over up to 16 workgroups
- * per token tile and their softmax partials merged by a second kernel. The
+ * kernel has one pass): workgroups that do not fill a round of the 256 CUs
+ * (a small eval's, or what is left past the whole rounds) split their key
+ * tiles over up to 16 workgroups per token tile where that pays, and their
+ * softmax partials are merged by a second kernel. The
  * result equals one pass up to fp32 summation order. ws_bytes from
  * cujev_ops_attention_ws_bytes (0 = no split for this shape; a smaller ws
  * also runs one pass). */
@@ -167,9 +168,8 @@ size_t cujev_ops_attention_ws_bytes(int N, int Hq, int Hkv, int P);
  * key-split partials in a static device array the library holds, one per
  * GPU, until the process ends. It calls no hipMalloc / hipFree. Limit: the
  * partials of one call must fit CUJEV_OPS_ATTN_NOALLOC_SCRATCH_BYTES; every
- * shape the kernel accepts does (splits x N x Hq <= 32768 rows of 258
- * floats, since the kernel needs Hq = 4 Hkv), and a larger need is rejected
- * with status 6. Every call on one GPU shares the array, so calls that
+ * shape the kernel accepts does (at most 256 workgroups' shares of 128 rows
+ * of 258 floats), and a larger need is rejected with status 6. Every call on one GPU shares the array, so calls that
  * overlap on one GPU (other streams, other threads) race; serialise them.
  * The stream must belong to the current device. */
 #define CUJEV_OPS_ATTN_NOALLOC_SCRATCH_BYTES 33816576u /* 32.25 MiB */
