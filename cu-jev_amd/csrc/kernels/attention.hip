@@ -233,6 +233,7 @@ __global__ __launch_bounds__(256) void attention_kernel(
     /* ---- key tiles: state [0,P) then own [own_lo, own_hi] (64-aligned) ---- */
     const int own_lo = own_base[n0];
     const int own_hi = min(n0 + QW, N) - 1;
+    const int last_base = own_base[own_hi]; /* the latest segment start in the tile */
     const int nst = (P + BK - 1) / BK;
     const int own_t0 = own_lo / BK;
     const int ntl_all = nst + own_hi / BK - own_t0 + 1;
@@ -349,7 +350,11 @@ __global__ __launch_bounds__(256) void attention_kernel(
         const int gi = i + tb; /* index in the full tile list */
         const bool own = gi >= nst;
         const int kbase = own ? (own_t0 + gi - nst) * BK : gi * BK;
-        if (own || kbase + BK > P) {
+        /* a tile that every row of this block sees whole needs no mask: the
+         * state's full tiles, and own tiles from the last segment's start up
+         * to the first row (all but the last one or two of a causal prefill,
+         * where masking each cost about a fifth of the loop) */
+        if (own ? kbase < last_base || kbase + BK - 1 > n0 : kbase + BK > P) {
             const int lo = own ? base_n : 0, hi = own ? n : P - 1;
             const int k8 = kbase + 8 * h;
 #pragma unroll
@@ -500,40 +505,62 @@ __global__ __launch_bounds__(256) void attention_kernel(
         step(last, i, sa0, sa1, sb0, sb1, 1, 0);
     }
 
-    /* ---- epilogue: normalise, gate, store ---- */
-    if (!qvalid)
-        return;
+    /* ---- epilogue: normalise, gate, store ----
+     * O^T leaves through this wave's quarter of the (now idle) tile buffers,
+     * as fp32 rows of 1 KiB per token with the 16-byte piece p of token t in
+     * slot p ^ t, so that the gate loads and the stores are whole rows. From
+     * the accumulators' layout (8 bytes of 32 tokens per instruction) they
+     * took 7.5 us of the 41 of a 1024-token prefill, the partials' stores
+     * 2.5-4 us. */
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+    const float inv = SPLIT ? 1.f : l_tot > 0.f ? 1.f / l_tot : 0.f;
+    unsigned char *ob = smem + wave * (QW * D * 4);
+    static_assert(4 * QW * D * 4 <= LDS_BYTES, "O staging");
+    const int nt = min(QW, N - n0);
+    const bf16 *g = gate + (size_t)n0 * gts + (size_t)head * ghs + 4 * lane;
+    constexpr int EB = 16; /* rows whose gate loads go out together */
+    bf16x4 gv[2][EB];
+    auto load_gate = [&](int i) {
+#pragma unroll
+        for (int t = 0; t < EB; t++)
+            gv[i][t] = *(const bf16x4 *)(g + (size_t)min(i * EB + t, nt - 1) * gts);
+    };
+    if constexpr (!SPLIT)
+        load_gate(0);
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++)
+#pragma unroll
+        for (int gq = 0; gq < 4; gq++) {
+            const floatx4 v = {o[dt][4 * gq] * inv, o[dt][4 * gq + 1] * inv,
+                               o[dt][4 * gq + 2] * inv, o[dt][4 * gq + 3] * inv};
+            *(floatx4 *)(ob + col * 1024 + (((8 * dt + 2 * gq + h) ^ col) << 4)) = v;
+        }
+    auto row = [&](int t) { return *(const floatx4 *)(ob + t * 1024 + ((lane ^ t) << 4)); };
     if constexpr (SPLIT) { /* the unnormalised partial; the merge gates it */
-        float *po = part.o + (size_t)prow * D;
-#pragma unroll
-        for (int dt = 0; dt < 8; dt++)
-#pragma unroll
-            for (int gq = 0; gq < 4; gq++)
-                *(float4 *)(po + 32 * dt + 8 * gq + 4 * h) =
-                    make_float4(o[dt][4 * gq], o[dt][4 * gq + 1], o[dt][4 * gq + 2],
-                                o[dt][4 * gq + 3]);
-        if (h == 0) {
+        if (qvalid && h == 0) {
             part.l[prow] = l_tot;
             part.mu[prow] = mu_run;
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        float *po = part.o + (size_t)(slot * SLOT_ROWS + wave * QW) * D + 4 * lane;
+#pragma unroll 8
+        for (int t = 0; t < nt; t++)
+            *(floatx4 *)(po + (size_t)t * D) = row(t);
         return;
     }
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    const bf16 *g = gate + (size_t)n * gts + (size_t)head * ghs;
-    bf16 *dst = out + ((size_t)n * Hq + head) * D;
+    load_gate(1);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bf16 *dst = out + ((size_t)n0 * Hq + head) * D + 4 * lane;
 #pragma unroll
-    for (int dt = 0; dt < 8; dt++) {
+    for (int t = 0; t < QW; t++) {
+        const floatx4 v = row(t);
+        const bf16x4 gt = gv[t / EB][t % EB];
+        bf16x4 r;
 #pragma unroll
-        for (int gq = 0; gq < 4; gq++) {
-            const int d0 = 32 * dt + 8 * gq + 4 * h;
-            bf16x4 gv = *(const bf16x4 *)(g + d0);
-            bf16x4 r;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                r[e] = f2bf(o[dt][4 * gq + e] * inv * sigmoid_f(bf2f(gv[e])));
-            *(bf16x4 *)(dst + d0) = r;
-        }
+        for (int e = 0; e < 4; e++)
+            r[e] = f2bf(v[e] * sigmoid_f(bf2f(gt[e])));
+        if (t < nt)
+            *(bf16x4 *)(dst + (size_t)t * Hq * D) = r;
     }
 }
 
