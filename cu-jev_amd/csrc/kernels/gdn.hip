@@ -470,18 +470,176 @@ DEV void rows_f32(const float *src, size_t rs, int L, int tid, int nthr, bf16 (*
     }
 }
 
+/* What the one-chunk form (ONE) reads and writes beside the chunk's inputs:
+ * the state every segment continues (NULL: zeros), the gate z, the norm and
+ * the layer's output rows. */
+struct OneChunk {
+    const float *S_in;
+    const bf16 *z;
+    int zs;
+    const float *nw;
+    float eps;
+    bf16 *y;
+};
+
+/* Steps 6 and 7 of the one-chunk form (see gdn_chunk_a_kernel, ONE): W and U
+ * staged in AT and the v rows' place (Vh), S's rows in sr. Every wave passes
+ * the same barriers. */
+DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int lane, int u, bool hact,
+                       int hv, int Hv, int t0, int L, bf16 (*Vh)[DK + 8], float (*AT)[CH + 4],
+                       const float *Gg, const float4 (&sr)[2][8], const bf16x8 (&qg)[4],
+                       const bf16x8 (&qkh)[2], const bf16x8 (&qkl)[2]) {
+    const int q4 = lane >> 4, c16 = lane & 15;
+    const bool act = hact && 16 * w4 < L; /* this wave's rows hold tokens */
+    bf16(*Wst)[DK + 8] = reinterpret_cast<bf16(*)[DK + 8]>(&AT[0][0]);
+    float(*Ust)[DV + 4] = reinterpret_cast<float(*)[DV + 4]>(&Vh[0][0]);
+    bf16x8 w[4];
+    floatx4 uf[8];
+    if (act) {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            w[s] = ld8(&Wst[16 * w4 + c16][32 * s + 8 * q4]);
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                uf[c][i] = Ust[16 * w4 + 4 * q4 + i][16 * c + c16];
+    }
+    lds_barrier(); /* W and U are in registers: their places are free */
+    /* S^T [column][dk], bf16, where U was */
+    bf16(*sT)[DK + 8] = Vh;
+    static_assert(sizeof(bf16) * DV * (DK + 8) <= 2 * sizeof(bf16) * CH * (DK + 8), "S^T");
+    if (hact) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            bf16x8 c[4];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                c[0][e] = f2bf(sr[i][e].x);
+                c[1][e] = f2bf(sr[i][e].y);
+                c[2][e] = f2bf(sr[i][e].z);
+                c[3][e] = f2bf(sr[i][e].w);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                *(bf16x8 *)&sT[4 * (u & 31) + j][64 * i + 8 * (u >> 5)] = c[j];
+        }
+    }
+    lds_barrier();
+    /* V'^T hi and lo [column][64 tokens], the first v-head's where K was, the
+     * second's where W was; 16-byte piece p of column c in slot p ^ (c/2 % 8) */
+    unsigned char *vT = hg ? (unsigned char *)&sm.AT[0][0][0] : (unsigned char *)&sm.Kh[0][0];
+    static_assert(2 * DV * CH * sizeof(bf16) <= 2 * sizeof(bf16) * CH * (DK + 8) &&
+                  2 * DV * CH * sizeof(bf16) <= sizeof(sm.AT), "V' staging");
+    constexpr int VLO = DV * CH * 2; /* bytes from the hi part to the lo part */
+    auto vslot = [](int col, int piece) { return col * (CH * 2) + ((piece ^ ((col >> 1) & 7)) << 4); };
+    floatx4 O[8];
+    float eg[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        eg[i] = hact ? fast_exp(Gg[16 * w4 + 4 * q4 + i]) : 0.f;
+    if (hact) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            bf16x4 ph = {}, pl = {}; /* rows without tokens: zero V' */
+            O[c] = floatx4{};
+            if (act) {
+                floatx4 V = {};
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    const bf16x8 sb = ld8(&sT[16 * c + c16][32 * s + 8 * q4]);
+                    V = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s], sb, V, 0, 0, 0);
+                    O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qg[s], sb, O[c], 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    O[c][i] *= eg[i];
+                    const bfpair sp = split2(uf[c][i] - V[i]);
+                    ph[i] = sp.hi;
+                    pl[i] = sp.lo;
+                }
+            }
+            unsigned char *d = vT + vslot(16 * c + c16, 2 * w4 + (q4 >> 1)) + 8 * (q4 & 1);
+            *(bf16x4 *)d = ph;
+            *(bf16x4 *)(d + VLO) = pl;
+        }
+    }
+    lds_barrier(); /* V' of every row; S^T is read */
+    float(*ob)[DV + 4] = reinterpret_cast<float(*)[DV + 4]>(&Vh[0][0]);
+    if (act) {
+        const int nks = (L + 31) >> 5;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                if (s >= nks)
+                    continue;
+                const unsigned char *v = vT + vslot(16 * c + c16, 4 * s + q4);
+                const bf16x8 vh_ = *(const bf16x8 *)v, vl_ = *(const bf16x8 *)(v + VLO);
+                O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkh[s], vh_, O[c], 0, 0, 0);
+                O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkh[s], vl_, O[c], 0, 0, 0);
+                O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkl[s], vh_, O[c], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                ob[16 * w4 + 4 * q4 + i][16 * c + c16] = O[c][i];
+        }
+    }
+    lds_barrier();
+    /* gated RMSNorm, 16 lanes per token row (as gdn_norm_gate_kernel) */
+    if (!hact)
+        return;
+    const int sl = u & 15;
+    float wl[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        wl[e] = one.nw[8 * sl + e];
+    for (int t = u >> 4; t < L; t += 16) { /* whole 16-lane groups */
+        const float4 o0 = *(const float4 *)&ob[t][8 * sl];
+        const float4 o1 = *(const float4 *)&ob[t][8 * sl + 4];
+        const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+        const size_t n = (size_t)t0 + t;
+        const bf16 *zr = one.z + n * one.zs + hv * DV + 8 * sl;
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            ss += ov[e] * ov[e];
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1)
+            ss += __shfl_xor(ss, m, 64);
+        const float inv = rsqrtf(ss * (1.f / DV) + one.eps);
+        bf16x8 res;
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            res[e] = f2bf(bf2f(f2bf(ov[e] * inv)) * wl[e] * silu_f(bf2f(zr[e])));
+        *(bf16x8 *)(one.y + (n * Hv + hv) * DV + 8 * sl) = res;
+    }
+}
+
+/* ONE: chunks that each hold whole segments with no state written back (eval
+ * branches). Nothing carries over between them, so the workgroup goes on to
+ * the outputs itself and none of phase B's operands leave the chip: with the
+ * masked QK^T and Q of its 16 rows held in registers as A fragments since
+ * step 3, and S^T (bf16) staged where the v rows were, wave w4 of each group
+ * computes rows 16 w4 .. +15 of
+ *   V' = U - W S (hi + lo, to LDS),  O = e^G (Q S) + QKm V'
+ * and the group applies the gated RMSNorm: the fragments, split products and
+ * order of operations of gdn_chunk_b_kernel and gdn_norm_gate_kernel, so the
+ * same bits. As two launches with the operands in memory between them (88 KiB
+ * a (chunk, v-head) out and 64 back), 64 branches x 16 of 32 v-heads took
+ * 30.4 + 18.6 us. */
 /* SRC 0: q, k, v, g, beta read from gdn_conv_prep's outputs (fp32); 1: computed
  * here from the pre-conv projection rows (zeros before a segment); 2: the
  * same with the state's conv tail before each segment. Grid: (chunk,
  * k-head x pairs of its v-heads); npairs = ceil(Hv / Hk / 2). */
-template <int SRC>
+template <int SRC, bool ONE>
 __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
     const float *__restrict__ qh, const float *__restrict__ kh_, const float *__restrict__ vh,
     const float *__restrict__ g, const float *__restrict__ beta, ConvSrc cv,
     const int32_t *__restrict__ chunk_tok0, const int32_t *__restrict__ chunk_len,
     const uint64_t *__restrict__ chunk_starts, int Hk, int Hv, int npairs,
     bf16 *__restrict__ Wo, bf16 *__restrict__ Qo, bf16 *__restrict__ QKo,
-    bf16 *__restrict__ KTo, float *__restrict__ Uo, float *__restrict__ Go) {
+    bf16 *__restrict__ KTo, float *__restrict__ Uo, float *__restrict__ Go, OneChunk one) {
     __shared__ PairA_Smem sm;
     const int ch = blockIdx.x, hk = blockIdx.y / npairs, pr = blockIdx.y - hk * npairs;
     const int rep = Hv / Hk;
@@ -571,7 +729,8 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
         sm.sV[r][lane] = bv;
         /* past the chunk's end g = 0: those lanes repeat the last token's G,
          * so G[63] is the chunk's total log-decay */
-        Go[((size_t)ch * Hv + hv) * 64 + lane] = gv;
+        if constexpr (!ONE)
+            Go[((size_t)ch * Hv + hv) * 64 + lane] = gv;
     }
     lds_barrier();
 
@@ -619,7 +778,7 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
                 }
             }
         }
-        if (wave >= 4 && pr == 0) { /* q rounded once: its hi part */
+        if (!ONE && wave >= 4 && pr == 0) { /* q rounded once: its hi part */
             const int u = tid - 256, t = u & 15, c8 = 32 * ((u >> 6) & 3) + 8 * ((u >> 4) & 3);
             const size_t ck = (size_t)ch * Hk + hk;
 #pragma unroll
@@ -645,6 +804,13 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
     /* token of accumulator slot r of 32-row tile tb */
     auto tok = [&](int tb, int r) { return 32 * tb + 8 * (r >> 2) + 4 * h + (r & 3); };
     const float *Gg = sm.G[hg];
+    const int q4 = lane >> 4, c16 = lane & 15;
+    bf16x8 qkh[2], qkl[2], qg[4]; /* ONE: QKm and Q of rows 16 w4 .. +15 */
+    if constexpr (ONE) {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            qg[s] = ld8(&sm.Xh[16 * w4 + c16][32 * s + 8 * q4]);
+    }
 
     /* ---- 3. per group (its v-head): masked QK^T hi + lo and A; the first
      * group of a k-head's first workgroup: K^T hi + lo for dk block 32 w4
@@ -657,7 +823,7 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
          * columns 32((i/64)%2) + 8((i/16)%4) .. +7 */
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const int i = u + 256 * j;
+            const int i = ONE ? 128 * w4 + 64 * j + lane : u + 256 * j;
             const int rr = 16 * (i >> 7) + (i & 15), c8 = 32 * ((i >> 6) & 1) + 8 * ((i >> 4) & 3);
             const float Gi = Gg[rr];
             const int Si = sm.Sid[rr];
@@ -672,8 +838,13 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
                 oh[e] = sp.hi;
                 ol[e] = sp.lo;
             }
-            *(bf16x8 *)(QKo + (cbg * 1024 + i) * 8) = oh;
-            *(bf16x8 *)(QKo + (cbg * 1024 + 512 + i) * 8) = ol;
+            if constexpr (ONE) {
+                qkh[j] = oh;
+                qkl[j] = ol;
+            } else {
+                *(bf16x8 *)(QKo + (cbg * 1024 + i) * 8) = oh;
+                *(bf16x8 *)(QKo + (cbg * 1024 + 512 + i) * 8) = ol;
+            }
         }
         /* A = tril(beta_i e^{G_i-G_j} k_i.k_j, -1) within a segment, zero
          * elsewhere (the inverse reads the upper part of its blocks): row
@@ -697,7 +868,7 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
             }
         }
     }
-    if (hg == 0 && pr == 0) {
+    if (!ONE && hg == 0 && pr == 0) {
         /* K^T as 32x32x16 A fragments (row dk = 32 w4 + l%32, tokens 16s +
          * 8(l/32)..+7) from the exact k rows (identity products of hi and
          * lo); the lane pair (l, l^32) trades halves */
@@ -834,6 +1005,7 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
 
     /* ---- 5. per group: W = T (beta e^G K) (dk block 32 w4, K hi) and
      * U = T (beta V) (dv block 32 w4, V hi + lo) ---- */
+    float4 sr[2][8]; /* ONE: S rows 64 i + 8 (u/32) .. +7, columns 4 (u%32) .. +3 */
     {
         const float *sKr = sm.sK[hg], *sVr = sm.sV[hg];
         floatx16 accw[2] = {}, accu[2] = {};
@@ -883,6 +1055,20 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
                 }
             }
         }
+        if constexpr (ONE) {
+            if (hact) { /* the state's columns, in flight under the staging */
+                const int u = tid & 255;
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        sr[i][e] = one.S_in ? *(const float4 *)(one.S_in +
+                                                                ((size_t)(hv0 + hg) * DK + 64 * i +
+                                                                 8 * (u >> 5) + e) * DV +
+                                                                4 * (u & 31))
+                                            : float4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         lds_barrier(); /* every wave is done with T and the v rows */
         if (hact) {
             bf16(*Wst)[DK + 8] = reinterpret_cast<bf16(*)[DK + 8]>(&AT[0][0]);
@@ -897,6 +1083,11 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
         }
     }
     lds_barrier();
+    if constexpr (ONE) {
+        one_chunk_out(sm, one, hg, w4, lane, tid & 255, hact, hv0 + hg, Hv, t0, L, Vh, AT, Gg, sr, qg,
+                      qkh, qkl);
+        return;
+    }
     /* ---- 6. W in the fragment order of Q; U (fp32) as 16x16
      * accumulator fragments: entry i = (32-column block i/256, row block
      * (i/64)%4, lane i%64) holds rows 16((i/64)%4) + 4((i/16)%4) + 0..3 of
@@ -1275,181 +1466,6 @@ __global__ __launch_bounds__(CB_THREADS) void gdn_chunk_b_kernel(
     }
 }
 
-/* ---------------------------------------------------------------------- */
-/* phase B for one-chunk segments with no state written back (eval branches) */
-/* ---------------------------------------------------------------------- */
-/* Every segment starts from the same S_in and nothing carries over between
- * them, so a workgroup takes one v-head and spw consecutive segments (as many
- * as keep about SB_WGS workgroups busy). Wave w (of 8: short per-wave chains,
- * since a few branches give few workgroups) owns state columns 16w..16w+15:
- * its S^T fragments (bf16) are read once into registers, then per segment it
- * computes those columns of
- *   V' = U - W S (hi + lo),  O = e^G (Q S) + QKm V'
- * for the 16-row blocks that hold tokens (the fragments and split products
- * of gdn_chunk_b_kernel), and the workgroup applies the gated RMSNorm of
- * gdn_norm_gate_kernel to the segment's fp32 rows. */
-constexpr int SB_WGS = 512;
-constexpr int SB_THREADS = 512; /* 8 waves, 16 state columns each */
-
-__global__ __launch_bounds__(SB_THREADS) void gdn_short_b_kernel(
-    const bf16x8 *__restrict__ Wi, const bf16x8 *__restrict__ Qi, const bf16x8 *__restrict__ QKi,
-    const float4 *__restrict__ Ui, const float *__restrict__ Gi,
-    const int32_t *__restrict__ chunk_tok0, const int32_t *__restrict__ chunk_len,
-    const int32_t *__restrict__ seg_chunk0, const int32_t *__restrict__ seg_nchunk, int nseg,
-    int spw, const float *__restrict__ S_in, int Hv, int Hk, const bf16 *__restrict__ z, int zs,
-    const float *__restrict__ nw, float eps, bf16 *__restrict__ y) {
-    /* S^T staging at the start, then each segment's fp32 O rows */
-    __shared__ __attribute__((aligned(16))) unsigned char so_raw[sizeof(bf16) * DV * (DK + 8)];
-    __shared__ __attribute__((aligned(16))) bf16 vTh[DV][CH + 8]; /* V'^T hi [column][token] */
-    __shared__ __attribute__((aligned(16))) bf16 vTl[DV][CH + 8]; /* V'^T lo                 */
-    bf16(*sT)[DK + 8] = reinterpret_cast<bf16(*)[DK + 8]>(so_raw);
-    float(*ob)[DV + 4] = reinterpret_cast<float(*)[DV + 4]>(so_raw);
-    static_assert(sizeof(float) * CH * (DV + 4) <= sizeof(bf16) * DV * (DK + 8), "O staging");
-
-    const int hv = blockIdx.y, sg0 = blockIdx.x * spw, hk = hv / (Hv / Hk);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int q4 = lane >> 4, c16 = lane & 15;
-    const int col0 = 16 * wave; /* this wave's 16 state columns */
-
-    /* S^T: thread reads S[dk0..dk0+7][dv4..dv4+3] (16-byte rows) and writes
-     * the 4 columns' 8-element runs */
-    {
-        const int dv4 = 4 * (tid & 31), dk0 = 8 * (tid >> 5);
-        float4 r[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            r[e] = S_in ? *(const float4 *)(S_in + ((size_t)hv * DK + dk0 + e) * DV + dv4)
-                        : float4{0.f, 0.f, 0.f, 0.f};
-        bf16x8 c[4];
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            c[0][e] = f2bf(r[e].x);
-            c[1][e] = f2bf(r[e].y);
-            c[2][e] = f2bf(r[e].z);
-            c[3][e] = f2bf(r[e].w);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            *(bf16x8 *)&sT[dv4 + j][dk0] = c[j];
-    }
-    /* V'^T rows past a segment's last 16-row block may be read by the QKm
-     * step (times an exact zero of the causal mask): keep them finite */
-    for (int i = tid; i < DV * (CH + 8) / 8; i += SB_THREADS) {
-        ((bf16x8 *)&vTh[0][0])[i] = bf16x8{};
-        ((bf16x8 *)&vTl[0][0])[i] = bf16x8{};
-    }
-    lds_barrier();
-    bf16x8 sb[4]; /* this wave's S^T fragments, the same for every segment */
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-        sb[s] = *(const bf16x8 *)&sT[col0 + c16][32 * s + 8 * q4];
-    lds_barrier(); /* sT's space now holds O */
-
-    float wl[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++)
-        wl[e] = nw[8 * (tid & 15) + e];
-
-    for (int j = 0; j < spw; j++) {
-        const int seg = sg0 + j;
-        if (seg >= nseg)
-            break;
-        /* without a segment table every unit is one (packed) chunk */
-        if (seg_chunk0 && seg_nchunk[seg] <= 0)
-            continue;
-        const int ch = seg_chunk0 ? seg_chunk0[seg] : seg;
-        const int t0 = chunk_tok0[ch], L = chunk_len[ch];
-        const int nrb = (L + 15) >> 4, nks = (L + 31) >> 5;
-        const size_t cb = (size_t)ch * Hv + hv, ck = (size_t)ch * Hk + hk;
-
-        floatx4 O[4];
-#pragma unroll
-        for (int rb = 0; rb < 4; rb++) {
-            O[rb] = floatx4{};
-            if (rb >= nrb)
-                continue;
-            bf16x8 w[4], qg[4];
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                w[s] = Wi[cb * 1024 + rb * 256 + 64 * s + lane];
-                qg[s] = Qi[ck * 1024 + rb * 256 + 64 * s + lane];
-            }
-            const float4 gq = *(const float4 *)(Gi + cb * 64 + 16 * rb + 4 * q4);
-            /* U fragment of the 32-column block holding these 16 columns:
-             * values 0..3 its first 16 columns, 4..7 the second */
-            const float4 *up = Ui + (cb * 1024 + ((wave >> 1) * 4 + rb) * 64 + lane) * 2;
-            const float4 uu = up[wave & 1];
-            floatx4 V = {};
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                V = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s], sb[s], V, 0, 0, 0);
-                O[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qg[s], sb[s], O[rb], 0, 0, 0);
-            }
-            /* O = e^G (Q S) + QKm V' */
-            O[rb][0] *= fast_exp(gq.x);
-            O[rb][1] *= fast_exp(gq.y);
-            O[rb][2] *= fast_exp(gq.z);
-            O[rb][3] *= fast_exp(gq.w);
-            const float uf[4] = {uu.x, uu.y, uu.z, uu.w};
-            bf16x4 ph, pl;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                { const bfpair sp_ = split2(uf[i] - V[i]); ph[i] = sp_.hi; pl[i] = sp_.lo; }
-            *(bf16x4 *)&vTh[col0 + c16][16 * rb + 4 * q4] = ph;
-            *(bf16x4 *)&vTl[col0 + c16][16 * rb + 4 * q4] = pl;
-        }
-        /* the wave reads back only its own columns of V'^T: LDS order suffices */
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int rb = 0; rb < 4; rb++) {
-            if (rb >= nrb)
-                continue;
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                if (s >= nks)
-                    continue;
-                const bf16x8 qkh = QKi[cb * 1024 + rb * 128 + 64 * s + lane];
-                const bf16x8 qkl = QKi[cb * 1024 + 512 + rb * 128 + 64 * s + lane];
-                const bf16x8 vh_ = *(const bf16x8 *)&vTh[col0 + c16][32 * s + 8 * q4];
-                const bf16x8 vl_ = *(const bf16x8 *)&vTl[col0 + c16][32 * s + 8 * q4];
-                O[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkh, vh_, O[rb], 0, 0, 0);
-                O[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkh, vl_, O[rb], 0, 0, 0);
-                O[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkl, vh_, O[rb], 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                ob[16 * rb + 4 * q4 + i][col0 + c16] = O[rb][i];
-        }
-        lds_barrier();
-        /* gated RMSNorm, 16 lanes per token row (as gdn_norm_gate_kernel) */
-        for (int r0 = 0; r0 < L; r0 += SB_THREADS / 16) {
-            const int t = r0 + (tid >> 4), sl = tid & 15;
-            if (t < L) { /* whole 16-lane groups */
-                const float4 o0 = *(const float4 *)&ob[t][8 * sl];
-                const float4 o1 = *(const float4 *)&ob[t][8 * sl + 4];
-                const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
-                const size_t n = (size_t)t0 + t;
-                const bf16 *zr = z + n * zs + hv * DV + 8 * sl;
-                float ss = 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-                    ss += ov[e] * ov[e];
-#pragma unroll
-                for (int m = 1; m < 16; m <<= 1)
-                    ss += __shfl_xor(ss, m, 64);
-                const float inv = rsqrtf(ss * (1.f / DV) + eps);
-                bf16x8 res;
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-                    res[e] = f2bf(bf2f(f2bf(ov[e] * inv)) * wl[e] * silu_f(bf2f(zr[e])));
-                *(bf16x8 *)(y + (n * Hv + hv) * DV + 8 * sl) = res;
-            }
-        }
-        lds_barrier(); /* ob and vT are rewritten by the next segment */
-    }
-}
-
 /* y = bf16( w * bf16(o * rsqrt(mean o^2 + eps)) * silu(z) ) from the fp32
  * output o: 16 lanes per (token, v-head) row, 8 columns a lane.
  * REF src/kernels/gdn.cu:193-216. */
@@ -1783,6 +1799,12 @@ extern "C" hipError_t k_gdn_conv_prep(const bf16_t *proj, int proj_stride, const
     return hipGetLastError();
 }
 
+/* Whether every chunk stands alone (packed whole segments, or one chunk per
+ * segment) and no state is written back: gdn_chunk_a_kernel's one-chunk form. */
+static bool one_chunk_segments(const cujev_chunks *ck, const float *S_out) {
+    return !S_out && (ck->chunk_starts || ck->max_seg_chunks == 1);
+}
+
 /* Phase B and the gated norm after phase A (either front end). */
 /* norm == false leaves o in ws->O for k_gdn_norm_gate (*o_pending = 1)
  * where a separate norm launch would follow; the short-segment kernel
@@ -1795,22 +1817,6 @@ static hipError_t gdn_phase_b(const cujev_chunks *ck, const float *S_in, float *
     if (o_pending)
         *o_pending = 0;
     const bool packed = ck->chunk_starts != nullptr;
-    if (!S_out && (packed || ck->max_seg_chunks == 1)) {
-        /* packed: the units are the chunks, each scanned from S_in */
-        const int units = packed ? ck->num_chunks : ck->num_segments;
-        const int spw = max(1, CEIL_DIV(units * Hv, SB_WGS));
-        if (tail.conv_out)
-            hipLaunchKernelGGL(gdn_conv_tail_kernel, dim3((unsigned)CEIL_DIV(tail.C, 256)),
-                               dim3(256), 0, stream, tail.proj, tail.ps, tail.conv_in,
-                               tail.conv_out, tail.seg0_len, tail.C);
-        hipLaunchKernelGGL(gdn_short_b_kernel, dim3((unsigned)CEIL_DIV(units, spw), (unsigned)Hv),
-                           dim3(SB_THREADS), 0, stream, (const bf16x8 *)ws->W, (const bf16x8 *)ws->Q,
-                           (const bf16x8 *)ws->QK, (const float4 *)ws->U, ws->G, ck->chunk_tok0,
-                           ck->chunk_len, packed ? nullptr : ck->seg_chunk0,
-                           packed ? nullptr : ck->seg_nchunk, units, spw, S_in, Hv, Hk,
-                           (const bf16 *)z, z_stride, norm_w, eps, (bf16 *)y);
-        return hipGetLastError();
-    }
     if (packed)
         return hipErrorInvalidValue; /* packed segments write no final state */
     const int units = ck->num_segments * Hv;
@@ -1838,10 +1844,15 @@ extern "C" hipError_t k_gdn_scan(const float *q, const float *k, const float *v,
     if (Hk <= 0 || Hv % Hk != 0 || (ck->chunk_starts && S_out))
         return hipErrorInvalidValue;
     const int npairs = CEIL_DIV(Hv / Hk, 2);
-    hipLaunchKernelGGL(gdn_chunk_a_kernel<0>, dim3((unsigned)ck->num_chunks, (unsigned)(Hk * npairs)),
+    const bool single = one_chunk_segments(ck, S_out);
+    const OneChunk one{S_in, (const bf16 *)z, z_stride, norm_w, eps, (bf16 *)y};
+    hipLaunchKernelGGL((single ? gdn_chunk_a_kernel<0, true> : gdn_chunk_a_kernel<0, false>),
+                       dim3((unsigned)ck->num_chunks, (unsigned)(Hk * npairs)),
                        dim3(PA_THREADS), 0, stream, q, k, v, g, beta, ConvSrc{}, ck->chunk_tok0,
                        ck->chunk_len, ck->chunk_starts, Hk, Hv, npairs, (bf16 *)ws->W, (bf16 *)ws->Q,
-                       (bf16 *)ws->QK, (bf16 *)ws->KT, ws->U, ws->G);
+                       (bf16 *)ws->QK, (bf16 *)ws->KT, ws->U, ws->G, one);
+    if (single)
+        return hipGetLastError();
     return gdn_phase_b(ck, S_in, S_out, z, z_stride, norm_w, eps, Hk, Hv, y, ws, N, TailJob{},
                        stream);
 }
@@ -1928,13 +1939,22 @@ static hipError_t gdn_layer(const bf16_t *proj, int proj_stride, const float *co
     /* the conv tail rides along with phase B */
     const TailJob tail{(const bf16 *)proj, proj_stride, conv_in, conv_out, seg0_len, C};
     const int npairs = CEIL_DIV(Hv / Hk, 2);
-    hipLaunchKernelGGL(conv_in ? gdn_chunk_a_kernel<2> : gdn_chunk_a_kernel<1>,
-                       dim3((unsigned)ck->num_chunks, (unsigned)(Hk * npairs)), dim3(PA_THREADS), 0,
-                       stream,
-                       (const float *)nullptr, (const float *)nullptr, (const float *)nullptr,
-                       (const float *)nullptr, (const float *)nullptr, cv, ck->chunk_tok0,
-                       ck->chunk_len, ck->chunk_starts, Hk, Hv, npairs, (bf16 *)ws->W,
-                       (bf16 *)ws->Q, (bf16 *)ws->QK, (bf16 *)ws->KT, ws->U, ws->G);
+    const bool single = one_chunk_segments(ck, S_out);
+    const OneChunk one{S_in, (const bf16 *)proj + C, proj_stride, norm_w, eps, (bf16 *)y};
+    auto kern = single ? (conv_in ? gdn_chunk_a_kernel<2, true> : gdn_chunk_a_kernel<1, true>)
+                       : (conv_in ? gdn_chunk_a_kernel<2, false> : gdn_chunk_a_kernel<1, false>);
+    if (single && conv_out) /* no phase B for the tail to ride along with */
+        hipLaunchKernelGGL(gdn_conv_tail_kernel, dim3((unsigned)CEIL_DIV(C, 256)), dim3(256), 0,
+                           stream, tail.proj, tail.ps, tail.conv_in, tail.conv_out, tail.seg0_len,
+                           tail.C);
+    hipLaunchKernelGGL(kern, dim3((unsigned)ck->num_chunks, (unsigned)(Hk * npairs)),
+                       dim3(PA_THREADS), 0, stream, (const float *)nullptr, (const float *)nullptr,
+                       (const float *)nullptr, (const float *)nullptr, (const float *)nullptr, cv,
+                       ck->chunk_tok0, ck->chunk_len, ck->chunk_starts, Hk, Hv, npairs,
+                       (bf16 *)ws->W, (bf16 *)ws->Q, (bf16 *)ws->QK, (bf16 *)ws->KT, ws->U, ws->G,
+                       one);
+    if (single)
+        return hipGetLastError();
     return gdn_phase_b(ck, S_in, S_out, proj + C, proj_stride, norm_w, eps, Hk, Hv, y, ws, N, tail,
                        stream, norm, o_pending);
 }
