@@ -58,6 +58,34 @@ constexpr int CH = 64;  /* chunk length   */
  * workgroup. Groups of head h < Hv also produce g and beta of v-head h. */
 constexpr int PREP_T = 8;
 
+/* Buffer resources over rows and states that a thread may have no part in:
+ * an offset past `bytes` reads as zero, so "this thread has no piece" and "no
+ * state was given" cost no branch. As conditional loads each became a branch,
+ * a load and a wait of its own: 16 trips to memory, one after the other. */
+DEV __amdgpu_buffer_rsrc_t in_rsrc(const void *base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+constexpr uint32_t OFF_NONE = 1u << 31; /* past the end of any of them, also with a row added */
+DEV bf16x8 in_ld8(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    return __builtin_bit_cast(bf16x8, v);
+}
+DEV float4 in_f4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
+                       __uint_as_float(v[3]));
+}
+DEV float in_f1(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+DEV bf16 in_bf(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(bf16, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+}
+/* v-head hv's state [DK][DV], or zeros */
+DEV __amdgpu_buffer_rsrc_t state_rsrc(const float *S, int hv) {
+    return in_rsrc(S + (S ? (size_t)hv * DK * DV : 0), S ? DK * DV * (uint32_t)sizeof(float) : 0u);
+}
+
 template <bool VEC, bool TAIL>
 __global__ __launch_bounds__(256) void gdn_conv_prep_kernel(
     const bf16 *__restrict__ proj, int ps, const float *__restrict__ conv_w,
@@ -311,22 +339,32 @@ struct TailJob {
     int seg0_len, C;
 };
 
-/* Conv weights and the state's tail (the same for every token block) of
- * `nsl` 128-channel slices starting at channel c0[sl] -> LDS:
+/* Conv weights and the state's tail (the same for every token block) of up to
+ * two 128-channel slices starting at channel c0[sl] -> LDS:
  * cw[(sl*8 + e)*16 + s] float4 and ct[(sl*3 + j)*128 + e*16 + s] for
- * channel 8s + e of slice sl. */
-template <bool TAIL>
-DEV void conv_stage(const ConvSrc &cv, const int *c0, int nsl, int tid, int nthr, float *cw,
-                    float *ct) {
-    for (int i = tid; i < nsl * DK; i += nthr) {
-        const int sl = i / DK, c = i % DK, cg = c0[sl] + c;
-        const int slot = (sl * 8 + (c & 7)) * 16 + (c >> 3);
-        *(float4 *)&cw[slot * 4] = *(const float4 *)(cv.conv_w + (size_t)cg * 4);
-        if constexpr (TAIL) {
+ * channel 8s + e of slice sl. In two halves over at least 256 threads, so that
+ * the loads go out with others and the LDS writes come later: a thread's
+ * channel (none past the slices), its weights and its tail. */
+struct ConvRegs {
+    float4 w;
+    float t[3];
+};
+template <bool TAIL> DEV void conv_load(const ConvSrc &cv, const int *c0, int nsl, int tid, ConvRegs &r) {
+    const int i = min(tid, nsl * DK - 1), cg = (i < DK ? c0[0] : c0[1]) + i % DK;
+    r.w = *(const float4 *)(cv.conv_w + (size_t)cg * 4);
 #pragma unroll
-            for (int j = 0; j < 3; j++)
-                ct[(sl * 3 + j) * 128 + (c & 7) * 16 + (c >> 3)] = cv.conv_in[(size_t)cg * 3 + j];
-        }
+    for (int j = 0; j < 3; j++)
+        r.t[j] = TAIL ? cv.conv_in[(size_t)cg * 3 + j] : 0.f;
+}
+template <bool TAIL> DEV void conv_store(const ConvRegs &r, int nsl, int tid, float *cw, float *ct) {
+    if (tid >= nsl * DK)
+        return;
+    const int sl = tid / DK, c = tid % DK;
+    *(float4 *)&cw[((sl * 8 + (c & 7)) * 16 + (c >> 3)) * 4] = r.w;
+    if constexpr (TAIL) {
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            ct[(sl * 3 + j) * 128 + (c & 7) * 16 + (c >> 3)] = r.t[j];
     }
 }
 
@@ -385,12 +423,12 @@ DEV void conv_slice(const bf16x8 (&x)[7], const int (&base)[4], const float *cw,
     const bool one_seg = base[0] == base[3];
     if (one_seg && n0 - 3 < base[0]) {
 #pragma unroll
-        for (int i = 0; i < 7; i++) {
-            const int k = n0 - 3 + i - base[0] + 3; /* tail slot of the row */
-            if (k < 3) {
+        for (int i = 0; i < 3; i++) { /* row 3 is token n0, in the segment */
+            const int k = n0 + i - base[0]; /* tail slot of the row, >= 0 */
 #pragma unroll
-                for (int e = 0; e < 8; e++)
-                    xf[i][e] = TAIL && k >= 0 ? ct[(sl * 3 + max(k, 0)) * 128 + e * 16 + s] : 0.f;
+            for (int e = 0; e < 8; e++) {
+                const float t = TAIL ? ct[(sl * 3 + min(k, 2)) * 128 + e * 16 + s] : 0.f;
+                xf[i][e] = k < 3 ? t : xf[i][e];
             }
         }
     }
@@ -476,18 +514,18 @@ DEV void rows_f32(const float *src, size_t rs, int L, int tid, int nthr, bf16 (*
 struct OneChunk {
     const float *S_in;
     const bf16 *z;
-    int zs;
+    int zs, zvec; /* row stride; whether z's 8-channel runs are 16-byte aligned */
     const float *nw;
     float eps;
     bf16 *y;
 };
 
 /* Steps 6 and 7 of the one-chunk form (see gdn_chunk_a_kernel, ONE): W and U
- * staged in AT and the v rows' place (Vh), S's rows in sr. Every wave passes
+ * staged in AT and the v rows' place (Vh), S^T's runs in sc. Every wave passes
  * the same barriers. */
 DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int lane, int u, bool hact,
                        int hv, int Hv, int t0, int L, bf16 (*Vh)[DK + 8], float (*AT)[CH + 4],
-                       const float *Gg, const float4 (&sr)[2][8], const bf16x8 (&qg)[4],
+                       const float *Gg, const bf16x8 (&sc)[2][4], const bf16x8 (&qg)[4],
                        const bf16x8 (&qkh)[2], const bf16x8 (&qkl)[2]) {
     const int q4 = lane >> 4, c16 = lane & 15;
     const bool act = hact && 16 * w4 < L; /* this wave's rows hold tokens */
@@ -511,19 +549,10 @@ DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int 
     static_assert(sizeof(bf16) * DV * (DK + 8) <= 2 * sizeof(bf16) * CH * (DK + 8), "S^T");
     if (hact) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            bf16x8 c[4];
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                c[0][e] = f2bf(sr[i][e].x);
-                c[1][e] = f2bf(sr[i][e].y);
-                c[2][e] = f2bf(sr[i][e].z);
-                c[3][e] = f2bf(sr[i][e].w);
-            }
+        for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                *(bf16x8 *)&sT[4 * (u & 31) + j][64 * i + 8 * (u >> 5)] = c[j];
-        }
+                *(bf16x8 *)&sT[4 * (u & 31) + j][64 * i + 8 * (u >> 5)] = sc[i][j];
     }
     lds_barrier();
     /* V'^T hi and lo [column][64 tokens], the first v-head's where K was, the
@@ -533,53 +562,80 @@ DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int 
                   2 * DV * CH * sizeof(bf16) <= sizeof(sm.AT), "V' staging");
     constexpr int VLO = DV * CH * 2; /* bytes from the hi part to the lo part */
     auto vslot = [](int col, int piece) { return col * (CH * 2) + ((piece ^ ((col >> 1) & 7)) << 4); };
-    floatx4 O[8];
-    float eg[4];
+    floatx4 O[8] = {};
+    bf16x4 ph[8] = {}, pl[8] = {}; /* rows without tokens: zero V' */
+    if (act) {
+        float eg[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        eg[i] = hact ? fast_exp(Gg[16 * w4 + 4 * q4 + i]) : 0.f;
+        for (int i = 0; i < 4; i++)
+            eg[i] = fast_exp(Gg[16 * w4 + 4 * q4 + i]);
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            floatx4 V = {};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const bf16x8 sb = ld8(&sT[16 * c + c16][32 * s + 8 * q4]);
+                V = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s], sb, V, 0, 0, 0);
+                O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qg[s], sb, O[c], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                O[c][i] *= eg[i];
+                const bfpair sp = split2(uf[c][i] - V[i]);
+                ph[c][i] = sp.hi;
+                pl[c][i] = sp.lo;
+            }
+        }
+    }
     if (hact) {
 #pragma unroll
         for (int c = 0; c < 8; c++) {
-            bf16x4 ph = {}, pl = {}; /* rows without tokens: zero V' */
-            O[c] = floatx4{};
-            if (act) {
-                floatx4 V = {};
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    const bf16x8 sb = ld8(&sT[16 * c + c16][32 * s + 8 * q4]);
-                    V = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s], sb, V, 0, 0, 0);
-                    O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qg[s], sb, O[c], 0, 0, 0);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    O[c][i] *= eg[i];
-                    const bfpair sp = split2(uf[c][i] - V[i]);
-                    ph[i] = sp.hi;
-                    pl[i] = sp.lo;
-                }
-            }
             unsigned char *d = vT + vslot(16 * c + c16, 2 * w4 + (q4 >> 1)) + 8 * (q4 & 1);
-            *(bf16x4 *)d = ph;
-            *(bf16x4 *)(d + VLO) = pl;
+            *(bf16x4 *)d = ph[c];
+            *(bf16x4 *)(d + VLO) = pl[c];
         }
+    }
+    /* the gates z of this thread's rows, under the QKm products */
+    const int sl = u & 15;
+    bf16x8 zv[4];
+    float wl[8];
+    if (hact) {
+        auto zrow = [&](int i) {
+            return one.z + (size_t)(t0 + min((u >> 4) + 16 * i, L - 1)) * one.zs + hv * DV + 8 * sl;
+        };
+        if (one.zvec) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                zv[i] = ld8(zrow(i));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    zv[i][e] = zrow(i)[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            wl[e] = one.nw[8 * sl + e];
     }
     lds_barrier(); /* V' of every row; S^T is read */
     float(*ob)[DV + 4] = reinterpret_cast<float(*)[DV + 4]>(&Vh[0][0]);
     if (act) {
-        const int nks = (L + 31) >> 5;
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
+        for (int s = 0; s < 2; s++) {
+            if (32 * s >= L)
+                break;
 #pragma unroll
-            for (int s = 0; s < 2; s++) {
-                if (s >= nks)
-                    continue;
+            for (int c = 0; c < 8; c++) {
                 const unsigned char *v = vT + vslot(16 * c + c16, 4 * s + q4);
                 const bf16x8 vh_ = *(const bf16x8 *)v, vl_ = *(const bf16x8 *)(v + VLO);
                 O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkh[s], vh_, O[c], 0, 0, 0);
                 O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkh[s], vl_, O[c], 0, 0, 0);
                 O[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qkl[s], vh_, O[c], 0, 0, 0);
             }
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 ob[16 * w4 + 4 * q4 + i][16 * c + c16] = O[c][i];
@@ -589,17 +645,15 @@ DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int 
     /* gated RMSNorm, 16 lanes per token row (as gdn_norm_gate_kernel) */
     if (!hact)
         return;
-    const int sl = u & 15;
-    float wl[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++)
-        wl[e] = one.nw[8 * sl + e];
-    for (int t = u >> 4; t < L; t += 16) { /* whole 16-lane groups */
+    for (int i = 0; i < 4; i++) {
+        const int t = (u >> 4) + 16 * i;
+        if (t >= L) /* whole 16-lane groups */
+            break;
         const float4 o0 = *(const float4 *)&ob[t][8 * sl];
         const float4 o1 = *(const float4 *)&ob[t][8 * sl + 4];
         const float ov[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
         const size_t n = (size_t)t0 + t;
-        const bf16 *zr = one.z + n * one.zs + hv * DV + 8 * sl;
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; e++)
@@ -611,7 +665,7 @@ DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int 
         bf16x8 res;
 #pragma unroll
         for (int e = 0; e < 8; e++)
-            res[e] = f2bf(bf2f(f2bf(ov[e] * inv)) * wl[e] * silu_f(bf2f(zr[e])));
+            res[e] = f2bf(bf2f(f2bf(ov[e] * inv)) * wl[e] * silu_f(bf2f(zv[i][e])));
         *(bf16x8 *)(one.y + (n * Hv + hv) * DV + 8 * sl) = res;
     }
 }
@@ -627,7 +681,17 @@ DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int 
  * order of operations of gdn_chunk_b_kernel and gdn_norm_gate_kernel, so the
  * same bits. As two launches with the operands in memory between them (88 KiB
  * a (chunk, v-head) out and 64 back), 64 branches x 16 of 32 v-heads took
- * 30.4 + 18.6 us. */
+ * 46.1 us, as one 36.5.
+ *
+ * One workgroup of two waves per SIMD fits a CU, and a chunk is a chain of
+ * steps between barriers, so what bounds either form is the latency inside
+ * each step: every trip to memory that waits for the one before costs 1-2 us,
+ * every LDS read that a branch keeps behind the previous product over 100
+ * cycles. So all of a step's loads go out before its first use (buffer loads
+ * that read zero where there is nothing to load, clamped indexes), and the
+ * masks and the kinds of products are selects or loops of their own, not
+ * branches inside an unrolled loop: 36.5 -> 28.5 us for those branches, a
+ * prefill of 2048 tokens 111.2 -> 104.9 us. */
 /* SRC 0: q, k, v, g, beta read from gdn_conv_prep's outputs (fp32); 1: computed
  * here from the pre-conv projection rows (zeros before a segment); 2: the
  * same with the state's conv tail before each segment. Grid: (chunk,
@@ -641,7 +705,17 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
     bf16 *__restrict__ Wo, bf16 *__restrict__ Qo, bf16 *__restrict__ QKo,
     bf16 *__restrict__ KTo, float *__restrict__ Uo, float *__restrict__ Go, OneChunk one) {
     __shared__ PairA_Smem sm;
-    const int ch = blockIdx.x, hk = blockIdx.y / npairs, pr = blockIdx.y - hk * npairs;
+    /* (k-head, pair) unit and chunk of this workgroup. Consecutive workgroups
+     * go to the 8 XCDs in turn: a unit's chunks stay on one of them, so its
+     * conv weights and (ONE) its state come from memory once, not once per
+     * XCD */
+    int ch = blockIdx.x, un = blockIdx.y;
+    if ((gridDim.y & 7) == 0) {
+        const int b = (int)(blockIdx.y * gridDim.x + blockIdx.x), i = b >> 3;
+        un = (b & 7) + 8 * (i / (int)gridDim.x);
+        ch = i % (int)gridDim.x;
+    }
+    const int hk = un / npairs, pr = un - hk * npairs;
     const int rep = Hv / Hk;
     const int hv0 = hk * rep + 2 * pr;   /* the pair's first v-head */
     const int nh = min(2, rep - 2 * pr); /* 1 or 2 v-heads */
@@ -665,7 +739,13 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
     float(*QK)[CH + 4] = reinterpret_cast<float(*)[CH + 4]>(&sm.Yl[0][0]);
     float(*AT)[CH + 4] = sm.AT[hg];
 
-    /* ---- 1. q and k rows (hi + lo); gates of the pair (waves 4, 5) ---- */
+    /* ---- 1. q and k rows (hi + lo); gates of the pair (waves 4, 5). Every
+     * global load of the steps up to 4 goes out here or, the v rows, in step
+     * 2: each further trip to memory inside the chain costs about 2 us. ---- */
+    bf16 gate_b = (bf16)0.f, gate_a = (bf16)0.f; /* waves 4, 5: token `lane`'s b and a */
+    float gate_A = 0.f, gate_dt = 0.f;
+    ConvRegs vw; /* the v-conv weights (and tail) of this thread's channel */
+    const int vc0[2] = {(2 * Hk + hv0) * DK, (2 * Hk + hv0 + 1) * DK};
     if constexpr (SRC == 0) {
         rows_f32(qh + ((size_t)t0 * Hk + hk) * DK, (size_t)Hk * DK, L, tid, PA_THREADS, sm.Xh,
                  sm.Xl);
@@ -685,8 +765,19 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
             for (int j = 0; j < 4; j++)
                 base[j] = cv.own_base[min(n0 + j, cv.N - 1)];
         }
+        {
+            const int hv = hv0 + min(max(wave - 4, 0), nh - 1);
+            const bf16 *ab = cv.proj + (size_t)min(t0 + lane, cv.N - 1) * cv.ps + C + Hv * DV;
+            gate_b = ab[hv];
+            gate_a = ab[Hv + hv];
+            gate_A = cv.A_neg_exp[hv];
+            gate_dt = cv.dt_bias[hv];
+        }
+        ConvRegs cw;
         const int c0s[2] = {hk * DK, (Hk + hk) * DK};
-        conv_stage<TAIL>(cv, c0s, 2, tid, PA_THREADS, sm.cs, sm.cs + 2 * 8 * 16 * 4);
+        conv_load<TAIL>(cv, c0s, 2, tid, cw);
+        conv_load<TAIL>(cv, vc0, nh, tid, vw);
+        conv_store<TAIL>(cw, 2, tid, sm.cs, sm.cs + 2 * 8 * 16 * 4);
         const int zrows = CH - 4 * nblk; /* rows of blocks without tokens: zeros */
         for (int i = tid; i < 4 * zrows * 16; i += PA_THREADS) {
             const int a = i / (zrows * 16), rem = i - a * zrows * 16;
@@ -711,9 +802,8 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
                 gv = g[(size_t)(t0 + lane) * Hv + hv];
                 bv = beta[(size_t)(t0 + lane) * Hv + hv];
             } else {
-                const bf16 *ab = cv.proj + (size_t)(t0 + lane) * cv.ps + C + Hv * DV;
-                bv = sigmoid_f(bf2f(ab[hv]));
-                gv = cv.A_neg_exp[hv] * softplus_f(bf2f(ab[Hv + hv]) + cv.dt_bias[hv]);
+                bv = sigmoid_f(bf2f(gate_b));
+                gv = gate_A * softplus_f(bf2f(gate_a) + gate_dt);
             }
         }
         /* st = first token of this lane's segment, en = its last */
@@ -760,22 +850,27 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
         const int job = wave < 3 ? wave : wave == 3 ? 0 : wave >= 6 ? wave - 5 : -1;
         floatx16 acc = {};
         const int ti = job == 0 ? 0 : 1, tj = job == 2 ? 1 : 0;
-        if (job >= 0) {
+        /* one loop per kind: with the kind asked inside, a step's operand reads
+         * wait for the step before */
+        if (isqk) {
 #pragma unroll
             for (int ks = 0; ks < DK / 16; ks++) {
                 const int c = 16 * ks + 8 * h;
                 const bf16x8 bkh = ld8(&sm.Kh[32 * tj + col][c]);
-                if (isqk) {
-                    const bf16x8 aqh = ld8(&sm.Xh[32 * ti + col][c]);
-                    const bf16x8 aql = ld8(&sm.Xl[32 * ti + col][c]);
-                    const bf16x8 bkl = ld8(&sm.Kl[32 * tj + col][c]);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aqh, bkh, acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aqh, bkl, acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aql, bkh, acc, 0, 0, 0);
-                } else {
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(&sm.Kh[32 * ti + col][c]),
-                                                                  bkh, acc, 0, 0, 0);
-                }
+                const bf16x8 aqh = ld8(&sm.Xh[32 * ti + col][c]);
+                const bf16x8 aql = ld8(&sm.Xl[32 * ti + col][c]);
+                const bf16x8 bkl = ld8(&sm.Kl[32 * tj + col][c]);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aqh, bkh, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aqh, bkl, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aql, bkh, acc, 0, 0, 0);
+            }
+        } else if (job >= 0) {
+#pragma unroll
+            for (int ks = 0; ks < DK / 16; ks++) {
+                const int c = 16 * ks + 8 * h;
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ld8(&sm.Kh[32 * ti + col][c]),
+                                                              ld8(&sm.Kh[32 * tj + col][c]), acc, 0,
+                                                              0, 0);
             }
         }
         if (!ONE && wave >= 4 && pr == 0) { /* q rounded once: its hi part */
@@ -827,14 +922,20 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
             const int rr = 16 * (i >> 7) + (i & 15), c8 = 32 * ((i >> 6) & 1) + 8 * ((i >> 4) & 3);
             const float Gi = Gg[rr];
             const int Si = sm.Sid[rr];
+            float Gj[8];
+            int Sj[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                Gj[e] = Gg[c8 + e], Sj[e] = sm.Sid[c8 + e];
             const float4 q0 = rd4(&QK[rr][c8]), q1 = rd4(&QK[rr][c8 + 4]);
             const float qv[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
             bf16x8 oh, ol;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const int cj = c8 + e;
-                const bool keep = rr >= cj && Si == sm.Sid[cj];
-                const bfpair sp = split2(keep ? qv[e] * fast_exp(fminf(Gi - Gg[cj], 0.f)) : 0.f);
+                const bool keep = (rr >= cj) & (Si == Sj[e]);
+                const float x = qv[e] * fast_exp(fminf(Gi - Gj[e], 0.f));
+                const bfpair sp = split2(keep ? x : 0.f);
                 oh[e] = sp.hi;
                 ol[e] = sp.lo;
             }
@@ -861,8 +962,10 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int cj = c16b + c4 + e;
-                    const bool keep = ri > cj && Si == sm.Sid[cj];
-                    a[e] = keep ? bi * kv[e] * fast_exp(fminf(Gi - Gg[cj], 0.f)) : 0.f;
+                    const int Sj = sm.Sid[cj];
+                    const bool keep = (ri > cj) & (Si == Sj);
+                    const float x = bi * kv[e] * fast_exp(fminf(Gi - Gg[cj], 0.f));
+                    a[e] = keep ? x : 0.f;
                 }
                 wr4(&AT[ri][c16b + c4], make_float4(a[0], a[1], a[2], a[3]));
             }
@@ -918,10 +1021,8 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
             }
         }
     }
-    if constexpr (CONV) {
-        int c0s[2] = {(2 * Hk + hv0) * DK, (2 * Hk + hv0 + 1) * DK};
-        conv_stage<SRC == 2>(cv, c0s, nh, tid, PA_THREADS, sm.cs, sm.cs + 2 * 8 * 16 * 4);
-    }
+    if constexpr (CONV) /* where the q and k slices' were */
+        conv_store<SRC == 2>(vw, nh, tid, sm.cs, sm.cs + 2 * 8 * 16 * 4);
     lds_barrier(); /* the q rows and the raw products are no longer read */
 
     /* ---- 4. the v rows of both v-heads (hi + lo) | T = (I + A)^-1 ----
@@ -964,8 +1065,7 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
         }
 #pragma unroll
         for (int i = 0; i < 16; i++)
-            if (i >= c)
-                AT[b0 + i][b0 + c] = t[i];
+            AT[b0 + i][b0 + c] = i >= c ? t[i] : 0.f; /* above the diagonal: 0 as it was */
     }
     lds_barrier();
     /* 4b: inside 32x32 diagonal block p (wave w4 = p): T_10 = -T_11 (A_10
@@ -1003,9 +1103,24 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
         lds_barrier();
     }
 
+    /* ONE: the state's rows 64 i + 8 (u/32) .. +7, columns 4 (u%32) .. +3 of
+     * this thread, in flight under the products; as S^T runs (column 4 (u%32) +
+     * j) once they are done. Loaded before the block steps they spill. */
+    float4 sr[2][8];
+    bf16x8 sc[2][4];
+    if constexpr (ONE) {
+        if (hact) {
+            const int u = tid & 255;
+            const __amdgpu_buffer_rsrc_t rs = state_rsrc(one.S_in, hv0 + hg);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    sr[i][e] = in_f4(rs, 4u * ((64 * i + 8 * (u >> 5) + e) * DV + 4 * (u & 31)));
+        }
+    }
     /* ---- 5. per group: W = T (beta e^G K) (dk block 32 w4, K hi) and
      * U = T (beta V) (dv block 32 w4, V hi + lo) ---- */
-    float4 sr[2][8]; /* ONE: S rows 64 i + 8 (u/32) .. +7, columns 4 (u%32) .. +3 */
     {
         const float *sKr = sm.sK[hg], *sVr = sm.sV[hg];
         floatx16 accw[2] = {}, accu[2] = {};
@@ -1056,17 +1171,22 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
             }
         }
         if constexpr (ONE) {
-            if (hact) { /* the state's columns, in flight under the staging */
-                const int u = tid & 255;
+            if (hact) {
 #pragma unroll
                 for (int i = 0; i < 2; i++)
 #pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        sr[i][e] = one.S_in ? *(const float4 *)(one.S_in +
-                                                                ((size_t)(hv0 + hg) * DK + 64 * i +
-                                                                 8 * (u >> 5) + e) * DV +
-                                                                4 * (u & 31))
-                                            : float4{0.f, 0.f, 0.f, 0.f};
+                    for (int e = 0; e < 8; e++) {
+                        sc[i][0][e] = f2bf(sr[i][e].x);
+                        sc[i][1][e] = f2bf(sr[i][e].y);
+                        sc[i][2][e] = f2bf(sr[i][e].z);
+                        sc[i][3][e] = f2bf(sr[i][e].w);
+                    }
+#pragma unroll
+                for (int i = 0; i < 8; i++) { /* rounded here, before the staging: 32 registers */
+                    u32x4 x = __builtin_bit_cast(u32x4, sc[i >> 2][i & 3]);
+                    asm volatile("" : "+v"(x));
+                    sc[i >> 2][i & 3] = __builtin_bit_cast(bf16x8, x);
+                }
             }
         }
         lds_barrier(); /* every wave is done with T and the v rows */
@@ -1084,7 +1204,7 @@ __global__ __launch_bounds__(PA_THREADS, 1) void gdn_chunk_a_kernel(
     }
     lds_barrier();
     if constexpr (ONE) {
-        one_chunk_out(sm, one, hg, w4, lane, tid & 255, hact, hv0 + hg, Hv, t0, L, Vh, AT, Gg, sr, qg,
+        one_chunk_out(sm, one, hg, w4, lane, tid & 255, hact, hv0 + hg, Hv, t0, L, Vh, AT, Gg, sc, qg,
                       qkh, qkl);
         return;
     }
@@ -1222,10 +1342,11 @@ __global__ __launch_bounds__(CB_THREADS) void gdn_chunk_b_kernel(
     if (wave < 4) {
         /* ---- chain waves: the recurrence ---- */
         floatx16 S; /* rows 32 w4 + 8(r/4) + 4h + r%4, column col0 + c32 */
+        const __amdgpu_buffer_rsrc_t rs = state_rsrc(S_in, hv);
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int dk = 32 * w4 + 8 * (r >> 2) + 4 * h + (r & 3);
-            S[r] = S_in ? S_in[((size_t)hv * DK + dk) * DV + col0 + c32] : 0.f;
+            S[r] = in_f1(rs, 4u * (dk * DV + col0 + c32));
         }
         /* consume S here, before any operand prefetch is in flight: S then
          * enters the chunk loop as a VALU result, and the loop's waits only
@@ -1484,7 +1605,10 @@ __global__ __launch_bounds__(CB_THREADS) void gdn_chunk_b_kernel(
  * the wave (one DPP rotate and two permlane swaps) and the token loop has no
  * barrier and no LDS traffic but the broadcast reads of k and q.
  * Before it, the workgroup stages the segment's pre-conv rows (its k-head's
- * q and k slices, its v columns) in LDS with every load in flight at once;
+ * q and k slices, its v columns) in LDS with every load in flight at once
+ * (as conditional loads they and the state's went out one after the other: 4
+ * branches x 20 of 32 v-heads took 17.4 us, 16.9 without those waits, 16.2
+ * with the conv's tokens four to a branch);
  * thread t then runs channel t's causal conv + SiLU over the tokens with
  * its weights and the state's tail in registers (gdn_conv_prep's
  * arithmetic), and 8 lanes per (token, q|k) row apply the l2-norm and q's
@@ -1531,9 +1655,8 @@ __global__ __launch_bounds__(RC_THREADS, 2) void gdn_recur_kernel(
     const int C = (2 * Hk + Hv) * DK;
     /* channel slot -> projection column: q slice, k slice, this block's v */
     auto gch = [&](int ch) {
-        return ch < DK       ? hk * DK + ch
-               : ch < 2 * DK ? (Hk + hk) * DK + ch - DK
-                             : (2 * Hk + hv) * DK + RC_COLS * cb + ch - 2 * DK;
+        const int kb = (Hk + hk - 1) * DK, vb = (2 * Hk + hv - 2) * DK + RC_COLS * cb;
+        return ch + (ch < DK ? hk * DK : ch < 2 * DK ? kb : vb);
     };
 
     /* ---- every global load first (one memory latency, not one per stage):
@@ -1541,21 +1664,17 @@ __global__ __launch_bounds__(RC_THREADS, 2) void gdn_recur_kernel(
      * conv weights and tail, and its slice of the state ---- */
     constexpr int XP = CEIL_DIV(RC_MAXL * (RC_CH / 8), RC_THREADS); /* row pieces per thread */
     const int npieces = L * (RC_CH / 8);
+    const __amdgpu_buffer_rsrc_t rows =
+        in_rsrc(cv.proj + (size_t)t0 * cv.ps, 2u * (uint32_t)L * (uint32_t)cv.ps);
     bf16x8 xr[XP];
 #pragma unroll
     for (int k = 0; k < XP; k++) {
         const int i = tid + k * RC_THREADS;
-        if (i < npieces) {
-            const int rr = i / (RC_CH / 8), ch = 8 * (i - rr * (RC_CH / 8));
-            xr[k] = ld8(cv.proj + (size_t)(t0 + rr) * cv.ps + gch(ch));
-        }
+        const int rr = i / (RC_CH / 8), ch = 8 * (i - rr * (RC_CH / 8));
+        xr[k] = in_ld8(rows, i < npieces ? 2u * (uint32_t)(rr * cv.ps + gch(ch)) : OFF_NONE);
     }
-    float b_raw = 0.f, a_raw = 0.f;
-    if (tid < L) {
-        const bf16 *ab = cv.proj + (size_t)(t0 + tid) * cv.ps + C + Hv * DV;
-        b_raw = bf2f(ab[hv]);
-        a_raw = bf2f(ab[Hv + hv]);
-    }
+    const uint32_t ab = tid < L ? 2u * (uint32_t)(tid * cv.ps + C + Hv * DV + hv) : OFF_NONE;
+    const float b_raw = bf2f(in_bf(rows, ab)), a_raw = bf2f(in_bf(rows, ab + 2u * Hv));
     const float A_neg = cv.A_neg_exp[hv], dtb = cv.dt_bias[hv];
     /* thread t convolves q/k channel t, and v channel t when t < RC_COLS */
     const int gq = gch(tid), gv = gch(2 * DK + (tid & (RC_COLS - 1)));
@@ -1569,9 +1688,10 @@ __global__ __launch_bounds__(RC_THREADS, 2) void gdn_recur_kernel(
     }
     const int c = lane & 7, r = lane >> 3, colw = 8 * wave + c;
     float S[16];
+    const __amdgpu_buffer_rsrc_t rs = state_rsrc(S_in, hv);
 #pragma unroll
     for (int i = 0; i < 16; i++)
-        S[i] = S_in ? S_in[((size_t)hv * DK + 16 * r + i) * DV + RC_COLS * cb + colw] : 0.f;
+        S[i] = in_f1(rs, 4u * ((16 * r + i) * DV + RC_COLS * cb + colw));
 #pragma unroll
     for (int k = 0; k < XP; k++) {
         const int i = tid + k * RC_THREADS;
@@ -1587,8 +1707,9 @@ __global__ __launch_bounds__(RC_THREADS, 2) void gdn_recur_kernel(
     lds_barrier();
 
     /* ---- conv + SiLU, a sliding window per channel: the channel's inputs
-     * of every row slot are read first (rows past L hold no token and are
-     * not used), so the window runs on registers ---- */
+     * of every row slot are read first (rows past L hold no token: what they
+     * give is written and not used), so the window runs on registers, four
+     * tokens between branches ---- */
     {
         float xin[RC_MAXL];
 #pragma unroll
@@ -1597,8 +1718,11 @@ __global__ __launch_bounds__(RC_THREADS, 2) void gdn_recur_kernel(
         float x3 = tq[0], x2 = tq[1], x1 = tq[2]; /* inputs of tokens -3, -2, -1 */
         float *dst = tid < DK ? &sm.q[0][tid] : &sm.k[0][tid - DK];
 #pragma unroll
-        for (int j = 0; j < RC_MAXL; j++) {
-            if (j < L) {
+        for (int j4 = 0; j4 < RC_MAXL; j4 += 4) {
+            if (j4 >= L)
+                break;
+#pragma unroll
+            for (int j = j4; j < j4 + 4; j++) {
                 const float x0 = xin[j];
                 float y = fmaf(wq.x, x3, 0.f);
                 y = fmaf(wq.y, x2, y);
@@ -1611,13 +1735,21 @@ __global__ __launch_bounds__(RC_THREADS, 2) void gdn_recur_kernel(
     }
     if (tid < 4 * RC_COLS) { /* v: channel tid % 32, token quarter tid / 32 */
         const int cc = tid & (RC_COLS - 1), per = (L + 3) >> 2;
-        const int j0 = (tid >> 5) * per, j1 = min(L, j0 + per);
+        const int j0 = (tid >> 5) * per; /* j0 + per <= RC_MAXL */
         auto xin = [&](int j) { /* input of token j, the tail before 0 */
             return j >= 0 ? bf2f(sm.x[j][2 * DK + cc]) : tv[j + 3];
         };
-        float x3 = xin(j0 - 3), x2 = xin(j0 - 2), x1 = xin(j0 - 1);
-        for (int j = j0; j < j1; j++) {
-            const float x0 = bf2f(sm.x[j][2 * DK + cc]);
+        static_assert(RC_MAXL % 4 == 0, "four quarters of the longest segment");
+        float x3 = xin(j0 - 3), x2 = xin(j0 - 2), x1 = xin(j0 - 1), xv[RC_MAXL / 4];
+#pragma unroll
+        for (int i = 0; i < RC_MAXL / 4; i++)
+            xv[i] = bf2f(sm.x[min(j0 + i, RC_MAXL - 1)][2 * DK + cc]);
+#pragma unroll
+        for (int i = 0; i < RC_MAXL / 4; i++) {
+            if (i >= per)
+                break;
+            const int j = j0 + i;
+            const float x0 = xv[i];
             float y = fmaf(wv.x, x3, 0.f);
             y = fmaf(wv.y, x2, y);
             y = fmaf(wv.z, x1, y);
@@ -1845,7 +1977,8 @@ extern "C" hipError_t k_gdn_scan(const float *q, const float *k, const float *v,
         return hipErrorInvalidValue;
     const int npairs = CEIL_DIV(Hv / Hk, 2);
     const bool single = one_chunk_segments(ck, S_out);
-    const OneChunk one{S_in, (const bf16 *)z, z_stride, norm_w, eps, (bf16 *)y};
+    const OneChunk one{S_in, (const bf16 *)z, z_stride,
+                       z_stride % 8 == 0 && ((uintptr_t)z & 15) == 0, norm_w, eps, (bf16 *)y};
     hipLaunchKernelGGL((single ? gdn_chunk_a_kernel<0, true> : gdn_chunk_a_kernel<0, false>),
                        dim3((unsigned)ck->num_chunks, (unsigned)(Hk * npairs)),
                        dim3(PA_THREADS), 0, stream, q, k, v, g, beta, ConvSrc{}, ck->chunk_tok0,
@@ -1940,7 +2073,7 @@ static hipError_t gdn_layer(const bf16_t *proj, int proj_stride, const float *co
     const TailJob tail{(const bf16 *)proj, proj_stride, conv_in, conv_out, seg0_len, C};
     const int npairs = CEIL_DIV(Hv / Hk, 2);
     const bool single = one_chunk_segments(ck, S_out);
-    const OneChunk one{S_in, (const bf16 *)proj + C, proj_stride, norm_w, eps, (bf16 *)y};
+    const OneChunk one{S_in, (const bf16 *)proj + C, proj_stride, 1, norm_w, eps, (bf16 *)y};
     auto kern = single ? (conv_in ? gdn_chunk_a_kernel<2, true> : gdn_chunk_a_kernel<1, true>)
                        : (conv_in ? gdn_chunk_a_kernel<2, false> : gdn_chunk_a_kernel<1, false>);
     if (single && conv_out) /* no phase B for the tail to ride along with */
