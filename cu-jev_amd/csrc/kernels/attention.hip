@@ -807,41 +807,63 @@ extern "C" hipError_t k_attn_prep_pair(const bf16_t *proj, int proj_stride,
     return hipGetLastError();
 }
 
+/* Shares per tile that `tiles` token tiles can have so that none waits for a
+ * CU: at most 256 workgroups, and where the XCDs are split among the kv-heads
+ * at most the 32 CUs of the XCD that serves most of them. 21 tiles of 4
+ * kv-heads 3 ways are 252 workgroups, but 33 on some XCDs: 44.6 us at 654
+ * tokens over 1160 keys, against 34.7 two ways and 38.7 in one pass. */
+static int max_shares(int tiles, int Hkv) {
+    int s = 256 / (tiles * Hkv);
+    if (8 % Hkv == 0) {
+        const int x = 32 / CEIL_DIV(tiles, 8 / Hkv);
+        s = s > x ? x : s;
+    }
+    return s > CUJEV_ATTN_MAX_SPLITS ? CUJEV_ATTN_MAX_SPLITS : s;
+}
+
 /* How a shape is shared out: token tiles 0 .. *full - 1 in launch order run
  * whole, the rest over the returned number of workgroups each (1: no split).
  * Whole rounds of 256 workgroups stay whole; what is left over (everything,
- * when there is less than one round) is split so that at most 256 workgroups
- * run it: at 64 branches x 40 over 8192 keys the last 64 of 320 workgroups
- * would otherwise hold a second round of 130 key tiles on a quarter of the
- * CUs. A split pays where the key tiles it takes off the longest share, at
- * about 1.5 us each, exceed the partials' write and read (0.3 us per MB) and
- * the merge launch (6 us); the smallest evals (N <= 256 tokens, under 128
- * workgroups) always split, as measured there. Every split needs at most 256
- * slots of partials. */
+ * when there is less than one round) is split where that pays: at 64 branches
+ * x 40 over 8192 keys the last 64 of 320 workgroups would otherwise hold a
+ * second round of 130 key tiles on a quarter of the CUs. The smallest evals
+ * (N <= 256 tokens, under 128 workgroups) always split, as measured there;
+ * past them the model below decides, fitted to 64 shapes with 1, 2 and 4
+ * kv-heads from 276 to 6179 tokens, each at up to 10 split counts: in us, one
+ * pass takes 10 and 1.27 a key tile; shares take 10-13 (the merge launch and
+ * the partials' latency), 0.035 a share for the partials' bytes, and 1.27 a
+ * key tile while under half the CUs work, up to 1.47 when all do. A split has
+ * to be 1.5 us better (4.5 with whole rounds before it: one launch more). Of
+ * the 64 none takes over 1.02 times one pass, and the pick is within 1.05
+ * times the best count except in five short ones (by up to 4 us). Every split
+ * needs at most 256 slots of partials. */
 extern "C" int cujev_attention_splits(int N, int Hkv, int P, int *full) {
     *full = 0;
     if (N <= 0 || P < 0 || Hkv <= 0)
         return 1;
     const int ntile = CEIL_DIV(N, QW);
-    /* at most as many shares as a token tile has key tiles (state + own) */
-    const int ntl_max = CEIL_DIV(P, BK) + CEIL_DIV(N, BK) + 1;
     if (N <= CUJEV_ATTN_SPLIT_MAX_N && ntile * Hkv < 128) {
-        int s = 256 / (ntile * Hkv);
+        /* at most as many shares as a token tile has key tiles (state + own) */
+        const int ntl_max = CEIL_DIV(P, BK) + CEIL_DIV(N, BK) + 1;
+        int s = max_shares(ntile, Hkv);
         s = s > ntl_max ? ntl_max : s;
-        s = s > CUJEV_ATTN_MAX_SPLITS ? CUJEV_ATTN_MAX_SPLITS : s;
         return s < 1 ? 1 : s;
     }
     const int nf = ntile * Hkv / 256 * 256 / Hkv; /* tiles of the whole rounds */
-    const int units = (ntile - nf) * Hkv;
+    const int left = ntile - nf, units = left * Hkv;
     if (units <= 0 || units > 128)
         return 1;
     /* key tiles of the longest leftover tile: the state and about two of its
      * own; with no state a causal prefill's, whose last positions are short */
-    const int len = P > 0 ? CEIL_DIV(P, BK) + 2 : (ntile - nf) * QW / BK + 1;
+    const int len = P > 0 ? CEIL_DIV(P, BK) + 2 : CEIL_DIV(N < left * QW ? N : left * QW, BK);
+    const int most = max_shares(left, Hkv);
     int best = 1;
-    double best_us = 1.5 * len;
-    for (int s = 2; s <= 256 / units && s <= CUJEV_ATTN_MAX_SPLITS && s <= len; s++) {
-        const double us = 1.5 * CEIL_DIV(len, s) + 6.0 + 0.3 * 0.132 * units * s;
+    const double merge_us = units < 33 ? 10.0 + 0.09 * units : 13.0;
+    double best_us = (P > 0 ? 10.0 : 8.5) + 0.025 * units + 1.27 * len - (nf > 0 ? 4.5 : 1.5);
+    for (int s = 2; s <= most && s <= len; s++) {
+        const int wgs = units * s;
+        const double tile_us = 1.27 + (wgs > 128 ? 0.2 * (wgs - 128) / 112 : 0.0);
+        const double us = merge_us + 0.035 * wgs + tile_us * CEIL_DIV(len, s);
         if (us < best_us)
             best_us = us, best = s;
     }

@@ -18,6 +18,8 @@ D = 256
     (12, 3, 1300, [50] * 8),            # Hkv not dividing 8, all shared
     (12, 3, 1984, [128] * 22),          # and 264 workgroups: 9 past 85 whole tiles
     (4, 1, 900, [7] * 100),             # one kv-head over the 8 XCDs
+    (16, 4, 1160, [4] * 163 + [2]),     # 21 tiles: 3 shares each would crowd an XCD
+    (16, 4, 700, [32] * 5),             # as would 12 of 5 tiles, in the smallest evals' rule
 ])
 def test_shared_key_tiles_equal_one_pass(Hq, Hkv, P, lens):
     from cujev import ops
