@@ -373,7 +373,11 @@ static double plan_us(int N, int M, int K, int gated, int RG, int NG, int S) {
 
 static int wide_plan(int N, int M, int K, int gated, int max_splits, int max_ng, int *RG, int *NG,
                      int *S) {
-    if (N <= 0 || M % 16 || K % GW_KC || (gated && M % 32))
+    /* X and W go through 32-bit buffer offsets: past 4 GiB there is no plan
+     * (the engine's 9B down projection past 174762 tokens), where the launch
+     * would refuse */
+    if (N <= 0 || M % 16 || K % GW_KC || (gated && M % 32) ||
+        (size_t)N * K * 2 > 0xffffffffull || (size_t)M * K * 2 > 0xffffffffull)
         return -1;
     const char *force = getenv("CUJEV_WIDE_PLAN");
     if (force) {

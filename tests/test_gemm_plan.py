@@ -25,3 +25,12 @@ def test_plan_rejects_unsupported_shapes():
     for N, M, K, gated in [(10, 100, 256, 0), (10, 256, 200, 0), (10, 272, 256, 1), (0, 256, 256, 0)]:
         with pytest.raises(o.OpsError):
             o.gemm_wide_plan(N, M, K, gated)
+
+
+def test_plan_ends_where_the_kernel_does():
+    """X of 4 GiB or more has no plan: the engine then takes hipBLASLt, while
+    the launch would be refused."""
+    o.load()
+    o.gemm_wide_plan(174762, 4096, 12288, False, 1)
+    with pytest.raises(o.OpsError):
+        o.gemm_wide_plan(174763, 4096, 12288, False, 1)
