@@ -444,7 +444,7 @@ def kernel_rooflines():
     gbr = gdn_roofline(case="gdn_branch")
     log(f"gdn config 2 branches: {gbr['us']:.1f} us, {gbr['gbs']:.1f} GB/s")
     res["gdn_branch_roofline"] = {"kernel": "gdn layer call: chunk_a (conv and gates inside, "
-                                            "packed chunks) + short_b (norm inside), config "
+                                            "packed chunks; V', O and norm inside), config "
                                             "2, 64 branches x 16 tokens", "bound": "hbm",
                                   "achieved": round(gbr["gbs"], 1), "peak": PEAK_HBM_GBS,
                                   "unit": "GB/s", "frac": round(gbr["gbs"] / PEAK_HBM_GBS, 4),
