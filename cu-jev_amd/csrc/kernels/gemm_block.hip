@@ -15,7 +15,9 @@
  *    token's row, its 16-byte pieces XOR-swizzled on the global side so that
  *    the fragment reads have no bank conflicts). No other vector memory
  *    operation is in flight in the loop, so the DMAs complete in order and a
- *    partial vmcnt wait covers them; one barrier per unit.
+ *    partial vmcnt wait covers them; one barrier per unit. Before it each wave
+ *    also waits for its LDS reads of what the unit's DMAs overwrite, a partial
+ *    lgkmcnt wait: gemm_block_order.h has the order and both counts.
  *  - The wave's own LDS reads run ahead of their MFMAs (X one unit, W three
  *    row groups), and at most one memory operation sits between two MFMAs:
  *    an MFMA leaves a wave about 3 issue slots, and reads and DMAs in bursts
@@ -46,6 +48,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_block_order.h"
 #include "kernels.h"
 
 namespace CUJEV_KNS {
@@ -75,7 +78,6 @@ DEV void gb_dma(__amdgpu_buffer_rsrc_t r, unsigned char *dst, uint32_t voff, uin
 }
 
 constexpr int GB_A = 256 * 64; /* bytes of a W unit: 256 rows x 32 k */
-constexpr int GB_WU = 4;       /* W units in the ring */
 
 template <int VM, int LGKM> DEV void gb_wait() {
     static_assert(VM < 64 && LGKM < 16, "counter ranges");
@@ -193,39 +195,36 @@ __global__ __launch_bounds__(256, 1) void gemm_block_kernel(
     gb_wait<WN + 4, 0>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    constexpr int AD = 3; /* W fragments read ahead, in rows */
     bf16x8 a[4], b0[WN], b1[WN];
 #pragma unroll
     for (int j = 0; j < WN; j++)
         b0[j] = rdb(0, j);
 #pragma unroll
-    for (int r = 0; r < AD; r++)
+    for (int r = 0; r < GB_AD; r++)
         a[r] = rda(0, r);
 
     /* unit u in ring slot S, its X fragments in b: reads unit u + 1's into bn */
     auto unit = [&](auto slot, int u, bf16x8 (&b)[WN], bf16x8 (&bn)[WN]) {
-        constexpr int S = decltype(slot)::value, SN = (S + 1) & 3, SP = (S + 3) & 3;
-        constexpr bool XD = S & 1;
-        gb_wait<XD ? 4 : 4 + WN, 4>();
+        constexpr int S = decltype(slot)::value;
+        gb_wait<gb_vm(S, WN), gb_lgkm(S, WN)>();
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        const int uw = min(u + 3, nu - 4 + SP), px = min((u >> 1) + 2, (nu >> 1) - 2 + (S >> 1));
+        const int uw = min(u + 3, nu - 4 + ((S + 3) & 3));
+        const int px = min((u >> 1) + 2, (nu >> 1) - 2 + (S >> 1));
 #pragma unroll
         for (int r = 0; r < 8; r++) {
-            const int jb = r * WN / 5, nbr = r < 5 ? (r + 1) * WN / 5 - jb : 0;
 #pragma unroll
             for (int j = 0; j < WN; j++) {
                 /* at most one memory operation between two MFMAs */
-                if (j == 0)
-                    a[(r + AD) & 3] = rda(r + AD < 8 ? S : SN, (r + AD) & 7);
-                if (j == 1 && XD && r < WN)
-                    dma_x(px, S >> 1, r);
-                if (j == 2 && nbr > 0)
-                    bn[jb] = rdb(SN, jb);
-                if (j == 3 && r >= 4)
-                    dma_w(uw, SP, r - 4);
-                if (j == (WN > 4 ? 4 : 3) && nbr > 1)
-                    bn[jb + 1] = rdb(SN, jb + 1);
+                const gb_mem m = gb_before(S, WN, r, j);
+                if (m.kind == GB_READ_A)
+                    a[m.row & 3] = rda(m.slot, m.row);
+                if (m.kind == GB_DMA_X)
+                    dma_x(px, m.slot >> 1, m.row);
+                if (m.kind == GB_READ_B)
+                    bn[m.row] = rdb(m.slot, m.row);
+                if (m.kind == GB_DMA_W)
+                    dma_w(uw, m.slot, m.row);
                 gb_mfma(acc[r][j], a[r & 3], b[j]);
                 __builtin_amdgcn_sched_barrier(0);
             }
