@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void attention_kernel(
     /* ---- key tiles: state [0,P) then own [own_lo, own_hi] (64-aligned) ---- */
     const int own_lo = own_base[n0];
     const int own_hi = min(n0 + QW, N) - 1;
-    const int last_base = own_base[own_hi]; /* the latest segment start in the tile */
+    int last_base = own_base[own_hi]; /* the last segment's start in the tile */
     const int nst = (P + BK - 1) / BK;
     const int own_t0 = own_lo / BK;
     const int ntl_all = nst + own_hi / BK - own_t0 + 1;
@@ -315,6 +315,11 @@ __global__ __launch_bounds__(256) void attention_kernel(
         issue_k(src_of(1), smem + K_OFF + K_BYTES, koff, wave);
     wait_tile_loads();
     __syncthreads();
+    /* a row that starts later still (bases that fall): no own tile goes unmasked.
+     * Asked here, where the rows' bases have arrived; per tile it cost 1 % of a
+     * 1024-token prefill */
+    if (__ballot(qvalid && base_n > last_base))
+        last_base = 0x7fffffff;
     floatx16 sa0 = floatx16{}, sa1 = floatx16{}, sb0, sb1;
 #pragma unroll
     for (int ks = 0; ks < 16; ks++) {

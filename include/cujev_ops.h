@@ -129,7 +129,10 @@ int cujev_op_attn_prep_pair(const void *proj, int proj_stride, const float *q_no
 
 /* Replaces reference src/kernels/kernels.h:203-206 (k_attention).
  * out bf16 [N][Hq*256] = sigmoid(gate) * softmax2(q.k) v over the state keys
- * [0,P) of (pk, pvt) and own keys [own_base[n], n] of (ok, ovt).
+ * [0,P) of (pk, pvt) and own keys [own_base[n], n] of (ok, ovt). 0 <=
+ * own_base[n] <= n, and of the 32 rows from a multiple of 32 on none starts
+ * before the first does (packed segments do not; a padding row that sees only
+ * itself may stand between a segment's rows, but not first of the 32).
  * gate element (n, h, d) is at gate[n*gate_tok_stride + h*gate_head_stride + d]. */
 int cujev_op_attention(const void *q, const void *gate, int gate_tok_stride, int gate_head_stride,
                        const void *pk, const void *pvt, int P, int p_stride, const void *ok,

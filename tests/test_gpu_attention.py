@@ -141,6 +141,28 @@ def test_attention_key_split_matches_oracle(seed, Hq, Hkv, P, seg_lens):
     assert e <= TOL and e1 <= 1e-2
 
 
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("P,seg_lens,pad", [
+    (0, [200], {70, 130, 131, 190}),          # amid a causal segment
+    (100, [160, 20, 60], {129, 150, 161, 201}),  # and beside segment starts
+])
+def test_attention_rows_that_see_only_themselves(P, seg_lens, pad, split):
+    """own_base[n] = n in rows that are neither the first nor the last of
+    their 32: the bases fall again behind them, and each row still sees
+    [own_base[n], n] only."""
+    o = ops()
+    Hq, Hkv = 8, 2
+    print(f"padding rows P={P} segs={seg_lens} pad={sorted(pad)} split={split}", flush=True)
+    q, gate, ks, vs, ko, vo, ob = make_case(61, Hq, Hkv, P, seg_lens)
+    for n in pad:
+        ob[n] = n
+    got, qd = run_attention(o, q, gate, ks, vs, ko, vo, ob, Hq, Hkv, split=split)
+    ref = oracle_attention(qd, gate, ks, vs, ko, vo, ob)
+    assert rel_err(got, ref) <= TOL
+    for n in pad:
+        assert rel_err(got[n], ref[n]) <= TOL, n
+
+
 @pytest.mark.parametrize("Hq,Hkv,Na,branches", [
     (16, 4, 530, [20] * 4),        # the deferred config-4 pass
     (8, 2, 17, [33, 1, 5]),
