@@ -595,11 +595,12 @@ DEV void one_chunk_out(PairA_Smem &sm, const OneChunk &one, int hg, int w4, int 
             *(bf16x4 *)(d + VLO) = pl[c];
         }
     }
-    /* the gates z of this thread's rows, under the QKm products */
+    /* the gates z of this thread's rows, under the QKm products (a chunk without
+     * tokens has no row to clamp to) */
     const int sl = u & 15;
     bf16x8 zv[4];
     float wl[8];
-    if (hact) {
+    if (hact && L > 0) {
         auto zrow = [&](int i) {
             return one.z + (size_t)(t0 + min((u >> 4) + 16 * i, L - 1)) * one.zs + hv * DV + 8 * sl;
         };

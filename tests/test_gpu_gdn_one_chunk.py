@@ -72,3 +72,34 @@ def test_one_launch_unaligned_operands(off, s_off):
         res.append(y.float().cpu().numpy())
     assert np.isfinite(res[1]).all()
     np.testing.assert_array_equal(res[0], res[1])
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_one_launch_chunks_without_tokens(packed):
+    """Chunks of length 0 (a table of a fixed size, a branch without tokens)
+    before, between and behind the others: nothing is read or written for
+    them, the other rows are the same bits."""
+    o = ops()
+    print(f"one chunk, empty chunks, packed={packed}", flush=True)
+    Hk, Hv, N, dev = 2, 4, 53, "cuda"
+    L = Layer(47, Hk, Hv)
+    pd = bf(L.proj(N)).to(dev)
+    t = lambda a, dt: torch.as_tensor(np.asarray(a, dt)).to(dev)
+    f = lambda a: t(a, np.float32)
+    base = t(np.repeat([0, 33], [33, 20]), np.int32)
+    cin, S = f(L.rng.standard_normal((L.C, 3))), f(L.rng.standard_normal((Hv, DK, DV)))
+    res = []
+    for tok0, clen in (([0, 33], [33, 20]), ([0, 0, 33, 33, 53], [0, 33, 0, 20, 0])):
+        n = len(tok0)
+        y = torch.full((N, Hv * DV), float("nan"), dtype=torch.bfloat16, device=dev)
+        scratch = torch.empty(o.gdn_scratch_bytes(n, Hv, N), dtype=torch.uint8, device=dev)
+        o.gdn_layer(pd, f(L.conv_w), cin, None, 0, base, f(L.A_neg), f(L.dt_bias),
+                    t(tok0, np.int32), t(clen, np.int32),
+                    None if packed else t(range(n), np.int32),
+                    None if packed else t([1] * n, np.int32), S, None, f(L.norm_w), L.eps, Hk, Hv,
+                    y, scratch, max_seg_chunks=1,
+                    chunk_starts=t([1] * n, np.int64) if packed else None)
+        torch.cuda.synchronize()
+        res.append(y.float().cpu().numpy())
+    assert np.isfinite(res[0]).all()
+    np.testing.assert_array_equal(res[1], res[0])
