@@ -58,13 +58,14 @@ typedef struct {
 /* Projection GEMMs Y[N,M] = X[N,K] W^T. For few tokens (the eval, N <= 96)
  * the hand-written weight-streaming kernel reads the pre-tiled copy of the
  * weight (its time is the HBM stream of W). Above that the hand-tiled kernels
- * (gemm_wide, gemm_block, same tiled copy) take every projection, at the tile
- * and K split cujev_gemm_plan picks: measured on MI355X against hipBLASLt's
- * heuristic choice on the plain rows, with cold weights, for the 4B and 9B
- * shapes at 13 token counts from 384 to 12288, 0.60-1.09 of its time (mean
- * 0.91) before the silu_mul launch that gate|up then also needs (101 us of
- * 956 at 10752 tokens). hipBLASLt is left for shapes the tiled copy does not
- * cover and for the LM head.
+ * (gemm_wide, gemm_block, same tiled copy) run at the tile and K split
+ * cujev_gemm_plan picks, except past 1000 tokens where the loaded hipBLASLt
+ * table was tuned for exactly the call's tokens and is the faster one
+ * (cujev_gemm_plan_loses, with the measurements). Sending those to the tiled
+ * kernels as well made the projections of a 4096-token 9B pass 1.04 times as
+ * long, of 12288 tokens 1.02 times; as it is none takes over 1.01 times
+ * hipBLASLt's time and most 0.90-0.99. hipBLASLt also takes the shapes that the
+ * tiled copy does not cover and the LM head.
  * CUJEV_SMALL_GEMM=0 / CUJEV_WIDE_GEMM=0 send those shapes to hipBLASLt. */
 static int env_on(const char *name) {
     const char *e = getenv(name);
@@ -85,12 +86,20 @@ static int wide_gemm_on(void) {
     return cached;
 }
 
+/* Whether the tiled kernels take a projection, and with which plan */
+static int tiled_gemm(cujev_model *m, int N, int M, int K, int gated, int max_splits, int *rg,
+                      int *ng, int *sp) {
+    return wide_gemm_on() && cujev_gemm_plan(N, M, K, gated, max_splits, rg, ng, sp) == 0 &&
+           !(cujev_gemm_plan_loses(N, K, gated, *rg, *ng, *sp) &&
+             cujev_gemm_tuned(m->gemm, N, M, K));
+}
+
 static hipError_t proj_gemm(cujev_model *m, const bf16_t *X, const bf16_t *W, const bf16_t *Wt,
                             bf16_t *Y, int N, int M, int K) {
     if (Wt && small_gemm_ok(N, M, K))
         return k_gemm_small(X, K, Wt, N, M, K, 0, 1, Y, M, NULL, m->stream);
     int rg, ng, sp;
-    if (Wt && wide_gemm_on() && cujev_gemm_plan(N, M, K, 0, 1, &rg, &ng, &sp) == 0)
+    if (Wt && tiled_gemm(m, N, M, K, 0, 1, &rg, &ng, &sp))
         return k_gemm_wide(X, K, Wt, N, M, K, 0, rg, ng, 1, Y, M, NULL, m->stream);
     return k_gemm(m->gemm, X, W, Y, 0, N, M, K, m->stream);
 }
@@ -114,11 +123,11 @@ static hipError_t resid_gemm(cujev_model *m, const bf16_t *X, const bf16_t *W, c
         }
         return k_gemm_small(X, K, Wt, N, M, K, 0, 1, m->y, M, NULL, m->stream);
     }
-    if (Wt && wide_gemm_on()) {
+    if (Wt) {
         size_t cap = m->ypart_bytes / ((size_t)N * M * 4);
         const int max_sp = cap > 8 ? 8 : cap < 1 ? 1 : (int)cap;
         int rg, ng, sp;
-        if (cujev_gemm_plan(N, M, K, 0, max_sp, &rg, &ng, &sp) == 0) {
+        if (tiled_gemm(m, N, M, K, 0, max_sp, &rg, &ng, &sp)) {
             if (sp > 1) {
                 *y = NULL;
                 *yp = m->ypart;
@@ -138,8 +147,7 @@ static hipError_t gate_up_gemm(cujev_model *m, const cujev_layer *ly, int N, int
         return k_gemm_small(m->xb, H, ly->wt_gate_up, N, 2 * I, H, 1, 1, m->act, I, NULL,
                             m->stream);
     int rg, ng, sp;
-    if (ly->wt_gate_up && wide_gemm_on() &&
-        cujev_gemm_plan(N, 2 * I, H, 1, 1, &rg, &ng, &sp) == 0)
+    if (ly->wt_gate_up && tiled_gemm(m, N, 2 * I, H, 1, 1, &rg, &ng, &sp))
         return k_gemm_wide(m->xb, H, ly->wt_gate_up, N, 2 * I, H, 1, rg, ng, 1, m->act, I, NULL,
                            m->stream);
     hipError_t e = proj_gemm(m, m->xb, ly->w_gate_up, NULL, m->proj, N, 2 * I, H);

@@ -264,6 +264,12 @@ extern "C" int cujev_gemm_version(cujev_gemm *g) {
     return v;
 }
 
+extern "C" int cujev_gemm_tuned(cujev_gemm *g, int N, int M, int K) {
+    std::lock_guard<std::mutex> lk(g->mu);
+    auto t = g->table.find(std::make_tuple(M, K, 0));
+    return t != g->table.end() && t->second.count(N) > 0;
+}
+
 /* Times every hipBLASLt solution that supports the problem (2 warm-up + 5
  * timed launches each, on the caller's buffers and stream; Y is rewritten)
  * and records the fastest in the table for this exact N. */

@@ -304,6 +304,9 @@ hipError_t k_gemm_small_tile(const bf16_t *W, int M, int K, bf16_t *Wt, hipStrea
  * plan. Tiles (4, 8) ungated, (4, 12) and (4, 16) run in gemm_block.hip. */
 int cujev_gemm_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
 int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
+/* 1 where hipBLASLt is faster than a plan, if it was tuned for exactly this
+ * shape (cujev_gemm_tuned). */
+int cujev_gemm_plan_loses(int N, int K, int gated, int RG, int NG, int S);
 /* k_gemm_wide's 256-row tiles (gemm_block.hip): 32 WN tokens, WN 4, 6 or 8;
  * _ok: whether X's rows can be loaded as 16-byte pieces. */
 int cujev_gemm_block_ok(const bf16_t *X, int ldx);
@@ -327,6 +330,8 @@ hipError_t k_gemm(cujev_gemm *g, const bf16_t *X, const bf16_t *W, void *Y, int 
  * -1 unreadable, -2 made with another hipBLASLt version. */
 int cujev_gemm_load_table(cujev_gemm *g, const char *path);
 int cujev_gemm_version(cujev_gemm *g);
+/* Whether the table has an algorithm for exactly (N, M, K), bf16 output. */
+int cujev_gemm_tuned(cujev_gemm *g, int N, int M, int K);
 /* Exhaustive hipBLASLt search for one shape; records the winner. */
 int cujev_gemm_tune(cujev_gemm *g, const bf16_t *X, const bf16_t *W, void *Y, int f32out, int N,
                     int M, int K, hipStream_t stream, int *best_index, float *best_us,
