@@ -10,9 +10,9 @@ eager prefill followed by an eval.
 
 Checked: fused evals against the eager engine and the float64 oracle, at
 state and branch lengths that straddle the 16/32-token query tiles, 64-key
-tiles and 64-token GDN chunks, with the GEMMs on the few-token, hand-tiled
-and hipBLASLt paths (the call's token count picks them) and with packed GDN
-chunks; the state left behind by a fused eval against an eager prefill's;
+tiles and 64-token GDN chunks, with the GEMMs on the few-token and hand-tiled
+paths (the call's token count picks them; the model's in_proj, whose rows the
+tiled copy does not cover, on hipBLASLt) and with packed GDN chunks; the state left behind by a fused eval against an eager prefill's;
 full-vocabulary logits; the =2 path bit for bit against eager; timing and
 argument checks. Bars as in test_gpu_engine.py: candidate probabilities
 within 3e-3 of the oracle (the engine's bf16 rounding points, and float64),

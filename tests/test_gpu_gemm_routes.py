@@ -1,7 +1,8 @@
 """Which kernels run an engine's projections past 96 tokens, seen from the
 hipBLASLt plans that a process prints as it makes them (CUJEV_GEMM_DEBUG): the
-tiled kernels by default, and hipBLASLt where its table was tuned for exactly the
-call's tokens. Results on every route within the engine tests' 3e-3 in probability of the default's,
+tiled kernels by default, hipBLASLt where its table was tuned for exactly the
+call's tokens, and hipBLASLt for all of them with CUJEV_WIDE_GEMM=0. Results
+on every route within the engine tests' 3e-3 in probability of the default's,
 and every repeat of an eval (eager, captured, replayed) the same bits.
 
 The switches are read once per process, so each route has a process of its own.
@@ -105,4 +106,15 @@ def test_an_entry_for_the_calls_tokens_goes_to_hipblaslt(model, default):
     x, plans = run(model, "tuned", CUJEV_GEMM_TABLE=str(table))
     big = {k: v for k, v in plans.items() if k[0] > 96 and k[1:] in projections(cfg)}
     assert big == {(N, qkv, H): "tuned table"}
+    assert np.abs(probabilities(x) - probabilities(default[0])).max() <= PROB_TOL
+
+
+def test_wide_gemm_off_runs_every_projection_on_hipblaslt(model, default):
+    """The fallback of shapes that the tiled copy does not cover: plain
+    projections, the residual ones and the unfused gate|up + silu_mul, in the
+    prefill of 200 tokens and the eval of 1056."""
+    cfg = model[1]
+    x, plans = run(model, "library", CUJEV_GEMM_TABLE="/nonexistent", CUJEV_WIDE_GEMM="0")
+    for n in (200, N):
+        assert {(m, k) for m_n, m, k in plans if m_n == n} >= projections(cfg)
     assert np.abs(probabilities(x) - probabilities(default[0])).max() <= PROB_TOL
