@@ -96,6 +96,13 @@ EXPORT int cujev_op_gemm_wide(const void *X, int ldx, const void *W, int N, int 
                     "gemm_wide");
 }
 
+EXPORT int cujev_ops_gemm_plan(int N, int M, int K, int gated, int max_splits, int *rg, int *ng,
+                               int *splits) {
+    if (!rg || !ng || !splits)
+        return -1;
+    return cujev_gemm_plan(N, M, K, gated, max_splits, rg, ng, splits);
+}
+
 EXPORT int cujev_ops_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *rg,
                                     int *ng, int *splits) {
     if (!rg || !ng || !splits)

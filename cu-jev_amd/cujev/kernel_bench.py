@@ -224,7 +224,7 @@ def wide_case(name, N=610):
     ops.load()
     M, K, gated = GEMM_SHAPES[name]
     residual = M <= 4096
-    rg, ng, sp = ops.gemm_wide_plan(N, M, K, gated, 8 if residual else 1)
+    rg, ng, sp = ops.gemm_plan(N, M, K, gated, 8 if residual else 1)
     dev = "cuda"
     ncopy = max(2, int(800e6 // (M * K * 2)) + 1)
     g = torch.Generator(device=dev).manual_seed(7)
@@ -274,8 +274,8 @@ def time_launches(launch, iters=20, warmup=3):
     return e0.elapsed_time(e1) / iters * 1e3
 
 
-WIDE_TILES = [(2, 8), (2, 12), (3, 8), (3, 12), (4, 6), (4, 8), (4, 10), (4, 12), (6, 4),
-              (6, 6), (6, 8), (8, 4), (8, 6)]
+WIDE_TILES = [(2, 8), (2, 12), (3, 8), (3, 12), (4, 6), (4, 8), (4, 10), (4, 12), (4, 16),
+              (6, 4), (6, 6), (6, 8), (8, 4), (8, 6)]
 
 
 def wide_sweep(token_counts, reps=15):

@@ -79,12 +79,16 @@ int cujev_ops_gemm_small_splits(int M, int K);
  * through a hand-tiled MFMA kernel. M % 16 == 0 (gated: M % 32 == 0),
  * K % 128 == 0, (K/128) % splits == 0, X and W under 4 GiB each. The tile is
  * 64 rg weight rows (gated: 32 rg gate rows and the same up rows) x 16 ng
- * tokens; (rg, ng) must be a pair cujev_ops_gemm_wide_plan can return, or
- * (4, 16). Every pair gives the same bits. */
+ * tokens; (rg, ng) must be a pair cujev_ops_gemm_plan can return. Every pair
+ * gives the same bits. */
 int cujev_op_gemm_wide(const void *X, int ldx, const void *W, int N, int M, int K, int gated,
                        int rg, int ng, int splits, void *Y, int ldy, float *P, void *stream);
-/* The best tile (rg, ng) of at most 192 tokens and split count (<=
- * max_splits) for a shape; 0 on success, -1 for an unsupported shape. */
+/* The tile (rg, ng) and split count (<= max_splits) that the engine's tiled
+ * kernels run a shape with; 0 on success, -1 for an unsupported shape. */
+int cujev_ops_gemm_plan(int N, int M, int K, int gated, int max_splits, int *rg, int *ng,
+                        int *splits);
+/* The same among the tiles of at most 192 tokens (from about 1000 tokens on
+ * the engine's, of up to 256, is the better one). */
 int cujev_ops_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *rg, int *ng,
                              int *splits);
 

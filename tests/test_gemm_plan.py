@@ -27,10 +27,28 @@ def test_plan_rejects_unsupported_shapes():
             o.gemm_wide_plan(N, M, K, gated)
 
 
-def test_plan_ends_where_the_kernel_does():
+@pytest.mark.parametrize("plan", [o.gemm_plan, o.gemm_wide_plan])
+def test_plan_ends_where_the_kernel_does(plan):
     """X of 4 GiB or more has no plan: the engine then takes hipBLASLt, while
     the launch would be refused."""
     o.load()
-    o.gemm_wide_plan(174762, 4096, 12288, False, 1)
+    plan(174762, 4096, 12288, False, 1)
     with pytest.raises(o.OpsError):
-        o.gemm_wide_plan(174763, 4096, 12288, False, 1)
+        plan(174763, 4096, 12288, False, 1)
+
+
+@pytest.mark.parametrize("M,K,gated,ms", [(10240, 2560, 0, 1), (18432, 2560, 1, 1),
+                                          (2560, 9216, 0, 8), (4096, 4096, 0, 8)])
+def test_engine_plan_takes_the_256_token_tile(M, K, gated, ms):
+    """The engine's planner may take one tile more than the other: where it
+    does not, they agree, and over many tokens it does."""
+    o.load()
+    taken = set()
+    for N in (1, 97, 305, 611, 1024, 2048, 4096, 6000, 8192, 10752, 12288):
+        p = o.gemm_plan(N, M, K, gated, ms)
+        if p[:2] == (4, 16):
+            taken.add(N)
+        else:
+            assert p == o.gemm_wide_plan(N, M, K, gated, ms)
+        assert 1 <= p[2] <= ms and (K // 128) % p[2] == 0
+    assert taken and min(taken) > 97
