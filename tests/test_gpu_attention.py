@@ -210,6 +210,43 @@ def test_attention_pair_equals_two_launches(Hq, Hkv, Na, branches):
     assert torch.equal(pair, two)
 
 
+@pytest.mark.parametrize("Hq,Hkv,Pa,Na,Pb,branches", [
+    (16, 4, 0, 530, 300, [20] * 4),        # b sees part of the state: a's rows are the longer
+    (8, 2, 700, 40, 64, [33, 1, 5]),       # a over more of the state than b
+    (12, 3, 129, 100, 0, [64, 7]),         # Hkv not dividing 8; b without state keys
+    (8, 2, 64, 33, 700, [70]),             # b first here
+])
+def test_attention_pair_in_either_order(Hq, Hkv, Pa, Na, Pb, branches):
+    """The paired launch starts the problem with the longer workgroups first.
+    Both orders, each problem with state keys and an own-key cache of its own:
+    the same bits as two one-pass launches."""
+    o = ops()
+    dev = "cuda"
+    Nb, P = int(sum(branches)), max(Pa, Pb)
+    N = Na + Nb
+    print(f"pair order Hq={Hq} Pa={Pa} Na={Na} Pb={Pb} branches={branches}", flush=True)
+    rng = np.random.default_rng(Na + Pb)
+    rnd = lambda *s: bf(rng.standard_normal(s)).to(dev)
+    cache = lambda n: (rnd(Hkv, o.kv_stride(n), D), rnd(Hkv, D, o.kv_stride(n)), o.kv_stride(n))
+    (pk, pvt, ps), (ak, avt, as_), (bk, bvt, bs) = cache(P), cache(Na), cache(Nb)
+    qd = bf(rng.standard_normal((N, Hq, D)) * 0.6 * orc.LOG2E / 16.0).to(dev)
+    gate = rnd(N, Hq, D)
+    starts = np.cumsum([0] + list(branches[:-1]))
+    base = np.concatenate([np.zeros(Na), np.repeat(starts, branches)]).astype(np.int32)
+    ob = torch.as_tensor(base).to(dev)
+    pair = torch.full((N, Hq * D), float("nan"), dtype=torch.bfloat16, device=dev)
+    o.attention_pair(qd, gate, Hq * D, D, pk, pvt, ps, ob, Hq, Hkv, pair, Na, Pa, ak, avt, as_,
+                     Pb, bk, bvt, bs)
+    two = torch.empty_like(pair)
+    o.attention(qd[:Na], gate[:Na], Hq * D, D, pk, pvt, Pa, ps, ak, avt, as_, ob[:Na], Hq, Hkv,
+                two[:Na])
+    o.attention(qd[Na:], gate[Na:], Hq * D, D, pk, pvt, Pb, ps, bk, bvt, bs, ob[Na:], Hq, Hkv,
+                two[Na:])
+    torch.cuda.synchronize()
+    assert torch.isfinite(pair.float()).all()
+    assert torch.equal(pair, two)
+
+
 def test_attention_branch_isolation():
     """A branch's output does not depend on its siblings. Not bit for bit:
     alone, the branch's rows sit at other positions of the 32-token tiles and
