@@ -1939,9 +1939,9 @@ static bool one_chunk_segments(const cujev_chunks *ck, const float *S_out) {
 }
 
 /* Phase B and the gated norm after phase A (either front end). */
-/* norm == false leaves o in ws->O for k_gdn_norm_gate (*o_pending = 1)
- * where a separate norm launch would follow; the short-segment kernel
- * applies the norm itself either way (*o_pending = 0). */
+/* norm == false leaves o in ws->O for k_gdn_norm_gate (*o_pending = 1). The
+ * one-chunk form does not come here (it applies the norm itself), so segments
+ * are not packed: those write no final state and always take it. */
 static hipError_t gdn_phase_b(const cujev_chunks *ck, const float *S_in, float *S_out,
                               const bf16_t *z, int z_stride, const float *norm_w, float eps,
                               int Hk, int Hv, bf16_t *y, const cujev_gdn_scratch *ws, int N,
@@ -1949,9 +1949,6 @@ static hipError_t gdn_phase_b(const cujev_chunks *ck, const float *S_in, float *
                               int *o_pending = nullptr) {
     if (o_pending)
         *o_pending = 0;
-    const bool packed = ck->chunk_starts != nullptr;
-    if (packed)
-        return hipErrorInvalidValue; /* packed segments write no final state */
     const int units = ck->num_segments * Hv;
     const int ntail = tail.conv_out ? CEIL_DIV(tail.C, CB_THREADS) : 0;
     hipLaunchKernelGGL(gdn_chunk_b_kernel, dim3((unsigned)(NCB * CEIL_DIV(units, 8) * 8 + ntail)),

@@ -324,7 +324,8 @@ hipError_t launch_mode(int WN, dim3 grid, hipStream_t s, const bf16 *X, int ldx,
     }
     CUJEV_GB_CASE(8)
     CUJEV_GB_CASE(6)
-    CUJEV_GB_CASE(4)
+    if constexpr (MODE != GB_GATED) /* gated 256 x 128 runs in gemm_wide.hip */
+        CUJEV_GB_CASE(4)
 #undef CUJEV_GB_CASE
     return hipErrorInvalidValue;
 }
