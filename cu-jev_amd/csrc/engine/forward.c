@@ -59,13 +59,12 @@ typedef struct {
  * the hand-written weight-streaming kernel reads the pre-tiled copy of the
  * weight (its time is the HBM stream of W). Above that the hand-tiled kernels
  * (gemm_wide, gemm_block, same tiled copy) run at the tile and K split
- * cujev_gemm_plan picks, except past 1000 tokens where the loaded hipBLASLt
+ * cujev_gemm_plan picks, except past 2048 tokens where the loaded hipBLASLt
  * table was tuned for exactly the call's tokens and is the faster one
- * (cujev_gemm_plan_loses, with the measurements). Sending those to the tiled
- * kernels as well made the projections of a 4096-token 9B pass 1.04 times as
- * long, of 12288 tokens 1.02 times; as it is none takes over 1.01 times
- * hipBLASLt's time and most 0.90-0.99. hipBLASLt also takes the shapes that the
- * tiled copy does not cover and the LM head.
+ * (cujev_gemm_plan_loses, with the measurements): with those on the tiled
+ * kernels as well, a 9B request of 8192 + 256 x 16 tokens took 153.1 ms against
+ * 150.4, with all of them on hipBLASLt 155.1. hipBLASLt also takes the shapes
+ * that the tiled copy does not cover and the LM head.
  * CUJEV_SMALL_GEMM=0 / CUJEV_WIDE_GEMM=0 send those shapes to hipBLASLt. */
 static int env_on(const char *name) {
     const char *e = getenv(name);
@@ -90,7 +89,7 @@ static int wide_gemm_on(void) {
 static int tiled_gemm(cujev_model *m, int N, int M, int K, int gated, int max_splits, int *rg,
                       int *ng, int *sp) {
     return wide_gemm_on() && cujev_gemm_plan(N, M, K, gated, max_splits, rg, ng, sp) == 0 &&
-           !(cujev_gemm_plan_loses(N, K, gated, *rg, *ng, *sp) &&
+           !(cujev_gemm_plan_loses(N, gated, *rg, *ng, *sp) &&
              cujev_gemm_tuned(m->gemm, N, M, K));
 }
 

@@ -415,26 +415,24 @@ extern "C" int cujev_gemm_plan(int N, int M, int K, int gated, int max_splits, i
 }
 
 /* Whether hipBLASLt runs this shape faster than the plan, given that its table
- * was tuned for exactly these tokens. Against such entries (4B and 9B shapes at
- * 1024 to 12288 tokens, cold weights, with the silu_mul or the residual add and
- * norm behind them):
- *  - ungated without a K split the plan took 0.94-1.22 of hipBLASLt's time,
- *    1.05 on average over 40 shapes: in_proj of 4B at 4096 tokens 248 us
- *    against 217, 9B down at 12288 907 / 858, 9B qkv at 8192 458 / 442;
- *  - with a split of 2048 k each (o_proj of 4B) 39.3 / 36.6 us at 1024 tokens
- *    and 41.4 / 39.5 at 1104; of 2304 k and more (down) 0.85-1.01;
- *  - gated, with the silu_mul launch that hipBLASLt then needs, 0.90-1.02 (9B at
- *    12288 tokens 1700 / 1721 us), but on this file's tiles past 2048 tokens
- *    338 / 328 us (4B at 4096).
- * For token counts it was not tuned for hipBLASLt runs a neighbour's algorithm,
- * and the plans take 0.90-1.00 of its time over a layer's projections. Up to
- * 1000 tokens they take 0.55-0.98 of it also where it was tuned. */
-extern "C" int cujev_gemm_plan_loses(int N, int K, int gated, int RG, int NG, int S) {
-    if (N <= 1000 || getenv("CUJEV_WIDE_PLAN"))
-        return 0;
-    if (gated)
-        return N > 2048 && !block_tile(RG, NG, 1);
-    return S == 1 || K / S <= 2048;
+ * was tuned for exactly these tokens. Against such entries of the 4B and 9B
+ * shapes (each projection by itself, cold weights, with the silu_mul or the
+ * residual add and norm behind it) the plan took, past 2048 tokens,
+ *  - ungated without a K split 0.98-1.22 of hipBLASLt's time, 1.06 on average
+ *    over 27 shapes: in_proj of 4B at 4096 tokens 248 us against 217, 9B down
+ *    at 12288 907 / 858, 9B qkv at 8192 458 / 442; with one (4B down at 2560)
+ *    1.01;
+ *  - gated, with the silu_mul launch that hipBLASLt then needs, 0.90-0.99 (9B
+ *    at 12288 tokens 1700 / 1721 us), but on this file's tiles 338 / 328 us (4B
+ *    at 4096).
+ * Up to 2048 tokens the plans are the faster ones inside a model, whatever the
+ * table has: prefills of 1024, 1104 and 1536 tokens through 8 layers of 4B, with
+ * an eval of 4, took 2.99, 3.18 and 3.93 ms with them and 3.03, 3.22 and 3.98
+ * with the entries (2048: 4.87 with either). For
+ * token counts without an entry hipBLASLt runs a neighbour's algorithm, and the
+ * plans take 0.90-1.00 of its time over a layer's projections. */
+extern "C" int cujev_gemm_plan_loses(int N, int gated, int RG, int NG, int S) {
+    return N > 2048 && (gated ? !block_tile(RG, NG, 1) : S == 1) && !getenv("CUJEV_WIDE_PLAN");
 }
 
 extern "C" hipError_t k_gemm_wide(const bf16_t *X, int ldx, const bf16_t *Wt, int N, int M, int K,

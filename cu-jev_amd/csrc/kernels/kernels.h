@@ -306,7 +306,7 @@ int cujev_gemm_plan(int N, int M, int K, int gated, int max_splits, int *RG, int
 int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
 /* 1 where hipBLASLt is faster than a plan, if it was tuned for exactly this
  * shape (cujev_gemm_tuned). */
-int cujev_gemm_plan_loses(int N, int K, int gated, int RG, int NG, int S);
+int cujev_gemm_plan_loses(int N, int gated, int RG, int NG, int S);
 /* k_gemm_wide's 256-row tiles (gemm_block.hip): 32 WN tokens, WN 4, 6 or 8;
  * _ok: whether X's rows can be loaded as 16-byte pieces. */
 int cujev_gemm_block_ok(const bf16_t *X, int ldx);

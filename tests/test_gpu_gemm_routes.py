@@ -23,8 +23,8 @@ from cujev import gemm_tune, ops, synthetic  # noqa: E402
 pytestmark = pytest.mark.gpu
 PROB_TOL = 3e-3
 PKG = Path(ops.__file__).resolve().parents[1]
-BRANCHES, LEN = 33, 32
-N = BRANCHES * LEN  # 1056 tokens: past the limit below which the tiled kernels always run
+BRANCHES, LEN = 33, 65
+N = BRANCHES * LEN  # 2145 tokens: past the limit below which the tiled kernels always run
 
 CHILD = """
 import sys
@@ -91,28 +91,32 @@ def test_tiled_kernels_run_without_an_entry(model, default):
 
 
 def test_an_entry_for_the_calls_tokens_goes_to_hipblaslt(model, default):
-    """qkv is tuned for N, in_proj for N + 32 only, gate|up for N: the first
-    runs on hipBLASLt, the second not (a neighbour's entry), nor the third
-    (the gated kernel is the faster one there)."""
+    """qkv, gate|up and out_proj are tuned for N, in_proj for N + 32 only. The
+    first runs on hipBLASLt, and gate|up, whose plan is not a 256-row tile of 192
+    tokens or more; not out_proj (its plan splits K), nor in_proj (a
+    neighbour's entry)."""
     d, cfg = model
     ops.load()
-    (qkv, H), _, (inp, _), _, (gu, _), _ = gemm_tune.projection_shapes(cfg)
+    (qkv, H), _, (inp, _), (_, vd), (gu, _), _ = gemm_tune.projection_shapes(cfg)
+    assert ops.gemm_plan(N, qkv, H)[2] == 1 and ops.gemm_plan(N, inp, H)[2] == 1
+    assert ops.gemm_plan(N, gu, H, True)[:2] not in {(4, 12), (4, 16)}
+    assert ops.gemm_plan(N, H, vd, False, 8)[2] > 1
     W = torch.randn(qkv, H, device="cuda").to(torch.bfloat16)
     X = torch.randn(N, H, device="cuda").to(torch.bfloat16)
     idx, _, _ = ops.gemm_tune(X, W, torch.empty(N, qkv, device="cuda", dtype=torch.bfloat16))
     table = d / "table.txt"
     table.write_text(f"# hipblaslt {ops.blaslt_version()}\n{N} {qkv} {H} 0 {idx}\n"
-                     f"{N + 32} {inp} {H} 0 {idx}\n{N} {gu} {H} 0 {idx}\n")
+                     f"{N + 32} {inp} {H} 0 {idx}\n{N} {gu} {H} 0 {idx}\n{N} {H} {vd} 0 {idx}\n")
     x, plans = run(model, "tuned", CUJEV_GEMM_TABLE=str(table))
-    big = {k: v for k, v in plans.items() if k[0] > 96 and k[1:] in projections(cfg)}
-    assert big == {(N, qkv, H): "tuned table"}
+    big = {k for k in plans if k[0] > 96 and k[1:] in projections(cfg)}
+    assert big == {(N, qkv, H), (N, gu, H)} and plans[(N, qkv, H)] == "tuned table"
     assert np.abs(probabilities(x) - probabilities(default[0])).max() <= PROB_TOL
 
 
 def test_wide_gemm_off_runs_every_projection_on_hipblaslt(model, default):
     """The fallback of shapes that the tiled copy does not cover: plain
     projections, the residual ones and the unfused gate|up + silu_mul, in the
-    prefill of 200 tokens and the eval of 1056."""
+    prefill of 200 tokens and the eval of 2145."""
     cfg = model[1]
     x, plans = run(model, "library", CUJEV_GEMM_TABLE="/nonexistent", CUJEV_WIDE_GEMM="0")
     for n in (200, N):
