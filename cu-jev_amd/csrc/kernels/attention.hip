@@ -835,13 +835,15 @@ static int max_shares(int tiles, int Hkv) {
  * (N <= 256 tokens, under 128 workgroups) always split, as measured there;
  * past them the model below decides, fitted to 64 shapes with 1, 2 and 4
  * kv-heads from 276 to 6179 tokens, each at up to 10 split counts: in us, one
- * pass takes 10 and 1.27 a key tile; shares take 10-13 (the merge launch and
- * the partials' latency), 0.035 a share for the partials' bytes, and 1.27 a
- * key tile while under half the CUs work, up to 1.47 when all do. A split has
- * to be 1.5 us better (4.5 with whole rounds before it: one launch more). Of
- * the 64 none takes over 1.02 times one pass, and the pick is within 1.05
- * times the best count except in five short ones (by up to 4 us). Every split
- * needs at most 256 slots of partials. */
+ * pass takes 10 (8.5 without a state), 0.025 a workgroup that could share and
+ * 1.27 a key tile; shares take 10 and 0.09 a workgroup of one pass, 13 from 33
+ * of those on (the merge launch and the partials' latency), 0.035 a share for
+ * the partials' bytes, and 1.27 a key tile while under half the CUs work, up to
+ * 1.50 when all do. A split has to be 1.5 us better (4.5 with whole rounds
+ * before it: one launch more). Timed at the rule's own picks none of the 64
+ * takes over 1.01 times one pass; 53 are within 1.05 times the best count, the
+ * worst at 1.16 (a prefill of 276 tokens, 2 us). Every split needs at most 256
+ * slots of partials. */
 extern "C" int cujev_attention_splits(int N, int Hkv, int P, int *full) {
     *full = 0;
     if (N <= 0 || P < 0 || Hkv <= 0)

@@ -40,11 +40,12 @@
  * unit, i.e. the matrix cores 1.6 PFLOP/s-equivalent (removing the DMAs gives
  * 1.63-1.67, the LDS reads as well 2.0: the clock under load and the LDS port
  * set the rest), plus about 8 us per round for launch, first loads and the
- * epilogue, and the last round's idle CUs. Measured against hipBLASLt
- * (untuned heuristic) at 10752 tokens: in_proj 512 against 590 us, gate|up +
- * silu 697 against 703 + 101, out_proj 163 / 162, down 387 / 347; against
- * gemm_wide's former (4, 8) at 611 tokens: qkv 37.6 / 41.6 us, in_proj 37.8 /
- * 41.2. */
+ * epilogue, and the last round's idle CUs. Measured for 4B at 10752 tokens
+ * against hipBLASLt with the nearest tuned entry (8832 tokens): in_proj 516 /
+ * 525 us, gate|up + silu 722 / 787, with the residual add and norm out_proj 237
+ * / 242 and down 457 / 478, but qkv 408 / 386; against entries tuned for the
+ * very count see cujev_gemm_plan_loses. Against gemm_wide's former (4, 8) at 611
+ * tokens: qkv 37.6 / 41.6 us, in_proj 37.8 / 41.2. */
 #include <type_traits>
 
 #include "common.h"

@@ -342,9 +342,10 @@ static int block_tile(int RG, int NG, int gated) {
  * the residual add's read of them (about 5 TB/s). For gemm_block's tiles the
  * measured time of a 32-k unit, which grows with the share of the CUs at
  * work (0.505-0.64 us at 256 tokens, 0.41-0.48 at 192, 0.355-0.42 at 128),
- * and a fixed 8 us per round (10 gated). Over the 4B and 9B shapes at 13 token
- * counts from 384 to 12288 the pick takes 1.02 times the measured best on
- * average and 1.14 at worst. */
+ * and a fixed 8 us per round (10 gated). Over the 4B and 9B shapes at 14 token
+ * counts from 384 to 12288, every tile and split timed, the pick takes 1.005
+ * times the measured best on average; of 140 picks five are over 1.05, the worst
+ * 1.13 (gate|up of 4B at 4096 tokens, (6, 8) 319 us against (4, 16) 281). */
 static double plan_us(int N, int M, int K, int gated, int RG, int NG, int S) {
     const int rows = gated ? M / 2 : M;
     const int bm = gated ? 32 * RG : 64 * RG;

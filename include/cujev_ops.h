@@ -176,8 +176,9 @@ size_t cujev_ops_attention_ws_bytes(int N, int Hq, int Hkv, int P);
  * GPU, until the process ends. It calls no hipMalloc / hipFree. Limit: the
  * partials of one call must fit CUJEV_OPS_ATTN_NOALLOC_SCRATCH_BYTES; every
  * shape the kernel accepts does (at most 256 workgroups' shares of 128 rows
- * of 258 floats), and a larger need is rejected with status 6. Every call on one GPU shares the array, so calls that
- * overlap on one GPU (other streams, other threads) race; serialise them.
+ * of 258 floats), and a larger need is rejected with status 6. Every call on
+ * one GPU shares the array, so calls that overlap on one GPU (other streams,
+ * other threads) race; serialise them.
  * The stream must belong to the current device. */
 #define CUJEV_OPS_ATTN_NOALLOC_SCRATCH_BYTES 33816576u /* 32.25 MiB */
 int cujev_op_attention_noalloc(const void *q, const void *gate, int gate_tok_stride,
@@ -210,8 +211,9 @@ size_t cujev_ops_gdn_scratch_bytes(int num_chunks, int Hv, int N);
  * S_out (may be NULL) = final state of segment 0. y bf16 [N][Hv*128] is the
  * gated-RMSNorm output; z is read at z[n*z_stride + hv*128 + c].
  * max_seg_chunks: the largest seg_nchunk entry as the caller knows it (0 =
- * not given); 1 with S_out == NULL (branches continuing a state) selects a
- * path that reads S once per v-head for a group of segments.
+ * not given); 1 with S_out == NULL (branches continuing a state) selects one
+ * launch for scan, output and norm, in which every chunk reads S for itself.
+ * A chunk may have length 0.
  * chunk_starts (device uint64 [num_chunks], may be NULL): packs several whole
  * segments of at most 64 tokens into one chunk; bit t is set where token t of
  * the chunk starts a segment. Only with S_out == NULL: every segment continues
