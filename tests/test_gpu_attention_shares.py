@@ -22,6 +22,18 @@ D = 256
     (16, 4, 700, [32] * 5),             # as would 12 of 5 tiles, in the smallest evals' rule
 ])
 def test_shared_key_tiles_equal_one_pass(Hq, Hkv, P, lens):
+    compare(Hq, Hkv, P, lens)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 17, 24, 25, 31, 32, 33])
+def test_partials_of_tiles_of_any_length(n):
+    """Partials leave row by row from another row in each wave: every row of a
+    tile of n tokens is written (the workspace is NaN until then)."""
+    compare(8, 2, 700, [n])
+
+
+def compare(Hq, Hkv, P, lens):
     from cujev import ops
     ops.load()
     N = sum(lens)
@@ -45,6 +57,7 @@ def test_shared_key_tiles_equal_one_pass(Hq, Hkv, P, lens):
         outs.append(out.float())
     assert torch.isfinite(outs[1]).all()
     assert float((outs[0] - outs[1]).abs().max()) <= 2 ** -8 * float(outs[0].abs().max())
+
 
 
 def test_partials_fit_the_static_scratch():
