@@ -300,7 +300,7 @@ hipError_t k_gemm_small_tile(const bf16_t *W, int M, int K, bf16_t *Wt, hipStrea
  * same up rows) x 16 NG tokens; cujev_gemm_plan picks RG, NG and a split
  * count <= max_splits (1 = no partials) for a shape and returns 0, or -1 for
  * an unsupported shape; cujev_gemm_wide_plan does so among the tiles of at
- * most 192 tokens (the operator ABI's). CUJEV_WIDE_PLAN="RG,NG,S" forces a
+ * most 192 tokens (the ABI has both). CUJEV_WIDE_PLAN="RG,NG,S" forces a
  * plan. Tiles (4, 8) ungated, (4, 12) and (4, 16) run in gemm_block.hip. */
 int cujev_gemm_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
 int cujev_gemm_wide_plan(int N, int M, int K, int gated, int max_splits, int *RG, int *NG, int *S);
